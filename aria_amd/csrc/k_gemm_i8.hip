@@ -17,8 +17,6 @@
  */
 #include "qgemm_dev.h"
 
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x16_t __attribute__((ext_vector_type(16)));
 
 /* ---- activation quantisation: one wave per row, the row held in registers ----
  * Lane l holds elements 4 (l + 64 j), j < nv = K / 256 (K % 256 == 0, up to 4096), or walks
@@ -353,10 +351,12 @@ extern "C" hipError_t aria_k_gemm_i8_t(void *y, int y_f16, const int8_t *xq, con
         hipLaunchKernelGGL(k_gemm_i8_simt, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
         return hipGetLastError();
     }
+    if (fm >= GEMM_KS) return qgemm_ks_launch(a, ARIA_WI8, fm - GEMM_KS, s);   /* the K-split kernel */
     if (fm >= 16) return qgemm_big_i8_launch(a, fm - 16, s);   /* the LDS-DMA kernel, configuration fm - 16 */
     const bool heads = a.epi.mode == ARIA_EPI_HEADS;
     if (fm <= 0 && K % 128 == 0 && (!heads || N <= 3072)) {
-        /* the LDS-DMA kernel (k_qgemm_big.hip) at every DiT shape: HEADS in 64 x 256, N <= 1024
+        /* the LDS-DMA kernel's (k_qgemm_big.hip) configurations at M = 2592, from which qgemm_pick
+         * (k_qgemm.hip) starts: HEADS in 64 x 256, N <= 1024
          * in 64 x 128, N <= 3072 in 128 x 128, wider in 192 x 128 (two workgroups per CU), except
          * N = 4096 in 192 x 256 tiles of 8 waves sharing the activation tile (ff_in 24.3 -> 23.6 us
          * with GELU, the same bits); N <= 1024
@@ -364,8 +364,10 @@ extern "C" hipError_t aria_k_gemm_i8_t(void *y, int y_f16, const int8_t *xq, con
          * pipelines (23.6 -> 21.7 us at K = 4096; at K = 1024 the split measured 6 % slower);
          * HEADS with N <= 1024 (ca_q: 164 tiles, one workgroup per busy CU) in 64 x 256 tiles
          * with the split (14.0 -> 12.7 us, the same bits: int32 sums are exact) */
-        return qgemm_big_i8_launch(a, heads ? ((N <= 1024 && (K / 128) % 2 == 0) ? 5 : 1) : N <= 1024 ? ((K >= 2048 && (K / 128) % 2 == 0) ? 4 : 0)
-                                                    : N <= 3072 ? 2 : N <= 4096 ? 6 : 3, s);
+        const int cur = heads ? ((N <= 1024 && (K / 128) % 2 == 0) ? 5 : 1)
+                      : N <= 1024 ? ((K >= 2048 && (K / 128) % 2 == 0) ? 4 : 0) : N <= 3072 ? 2 : N <= 4096 ? 6 : 3;
+        const int c = qgemm_pick(ARIA_WI8, heads, M, N, K, cur);
+        return c >= GEMM_KS ? qgemm_ks_launch(a, ARIA_WI8, c - GEMM_KS, s) : qgemm_big_i8_launch(a, c, s);
     }
     if (fm <= 0) {
         /* tile rows, from a sweep at M = 2592 (fm: 1..4 = 32..128 rows): 128 rows when those

@@ -381,6 +381,72 @@ static int pick_wr(int M, int N, int K) {
     return best;
 }
 
+/* ---- which kernel and tile: a launch costs about c0 + n (c1 + ck K / 1024) us, n = the tiles on
+ * the busiest of the 256 CUs. The constants are least-squares fits per configuration to a sweep of
+ * M = 40 .. 2592 over the DiT's projections (N / K = 1024 / 1024, 3072 / 1024, 4096 / 1024,
+ * 8192 / 1024, 1024 / 4096), each launch alone in a replayed graph over six operand sets; rms
+ * error 5-9 %. A candidate displaces the configuration that M = 2592 takes only where it is
+ * predicted 5 % faster. Over the sweep the picks run 1.64x (Q8, Q4), 1.24x (fp16), 1.52x (int8),
+ * HEADS 1.6-1.9x faster than those configurations in the geometric mean and are within 1-2 % of
+ * the fastest of each shape on average (fp16 4 %). Down to two rows of tiles the small tiles of
+ * k_qgemm_ks.hip win because they give every CU work; from about M = 860 (N = 8192) to 1420
+ * (N = 1024) on, the large tiles' fewer bytes per product do. */
+struct TileCost { int pick, bm, bn; float c0, c1, ck; };
+static const TileCost cost_q8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 1.4f}, {GEMM_KS + 1, 32, 64, 1.2f, 1.7f, 2.0f},
+    {GEMM_KS + 2, 64, 64, 1.3f, 3.2f, 2.6f}, {GEMM_KS + 3, 96, 64, 2.0f, 3.9f, 3.2f}, {GEMM_KS + 4, 64, 64, 2.9f, 0.6f, 3.4f},
+    {0, 96, 128, 2.5f, 3.4f, 5.5f}, {1, 128, 128, 3.2f, 3.8f, 6.5f}, {4, 224, 128, 8.7f, 6.4f, 6.4f},
+    {5, 96, 128, -0.5f, 7.1f, 4.9f}, {7, 192, 256, -4.8f, 14.9f, 14.9f}};
+static const TileCost cost_q4[] = {{GEMM_KS, 32, 32, 0.9f, 1.5f, 1.8f}, {GEMM_KS + 1, 32, 64, 1.1f, 1.7f, 2.7f},
+    {GEMM_KS + 2, 64, 64, 1.5f, 3.3f, 3.1f}, {GEMM_KS + 3, 96, 64, 1.8f, 3.6f, 4.0f}, {GEMM_KS + 4, 64, 64, 3.4f, 0.0f, 4.6f},
+    {0, 96, 128, 3.0f, 2.7f, 7.0f}, {1, 128, 128, 3.2f, 3.4f, 7.9f}, {4, 224, 128, 7.9f, 7.1f, 7.1f},
+    {5, 96, 128, -0.3f, 6.9f, 6.3f}, {7, 192, 256, -6.2f, 16.3f, 16.3f}};
+static const TileCost cost_f16[] = {{GEMM_KS, 32, 32, 1.1f, 1.6f, 1.5f}, {GEMM_KS + 1, 32, 64, 1.3f, 1.9f, 2.1f},
+    {GEMM_KS + 2, 64, 64, 1.3f, 3.0f, 2.8f}, {0, 64, 128, 1.6f, 2.4f, 5.4f}, {1, 96, 128, 4.1f, 0.7f, 8.6f},
+    {2, 128, 128, 5.0f, 1.0f, 9.9f}, {3, 160, 128, 6.1f, 0.7f, 11.2f}, {4, 192, 128, 6.8f, 1.6f, 12.0f}};
+static const TileCost cost_i8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 0.8f}, {GEMM_KS + 1, 32, 64, 0.9f, 2.2f, 1.1f},
+    {GEMM_KS + 2, 64, 64, 0.9f, 3.4f, 1.4f}, {GEMM_KS + 3, 96, 64, 1.4f, 4.1f, 1.9f}, {0, 64, 128, 2.0f, 3.1f, 2.2f},
+    {2, 128, 128, 5.1f, 1.3f, 4.9f}, {3, 192, 128, 6.6f, 2.3f, 5.7f}, {4, 96, 128, -0.2f, 6.1f, 3.4f},
+    {6, 192, 256, -6.7f, 12.3f, 12.3f}};
+/* HEADS (64 columns in one wave; timed at K = 1024 only, N = 1024 and 3072) */
+static const TileCost cost_q8_heads[] = {{GEMM_KS + 1, 32, 64, 1.1f, 2.4f, 2.0f}, {GEMM_KS + 3, 96, 64, 2.0f, 5.4f, 3.2f},
+    {GEMM_KS + 4, 64, 64, 3.5f, 1.2f, 3.4f}, {6, 64, 256, 1.0f, 8.0f, 6.2f}, {8, 64, 512, 7.7f, 6.0f, 9.4f}};
+static const TileCost cost_f16_heads[] = {{GEMM_KS + 1, 32, 64, 1.4f, 2.4f, 2.1f}, {GEMM_KS + 2, 64, 64, 1.3f, 4.1f, 2.8f},
+    {GEMM_KS + 3, 96, 64, 1.7f, 5.2f, 3.6f}, {GEMM_KS + 4, 64, 64, 3.5f, 1.4f, 3.6f}};
+static const TileCost cost_i8_heads[] = {{GEMM_KS + 1, 32, 64, 0.8f, 2.7f, 1.1f}, {GEMM_KS + 2, 64, 64, 0.9f, 4.3f, 1.4f},
+    {GEMM_KS + 3, 96, 64, 1.8f, 5.1f, 1.9f}, {GEMM_KS + 4, 64, 64, 3.4f, 1.5f, 1.9f}, {1, 64, 256, 12.3f, 0.9f, 2.2f},
+    {5, 64, 256, 3.0f, 6.2f, 4.0f}};
+
+int qgemm_pick(int wt, bool heads, int M, int N, int K, int cur) {
+    struct Table { const TileCost *t; int n; };
+#define TBL(x) Table{x, (int)(sizeof x / sizeof x[0])}
+    const Table tb = wt == ARIA_WI8 ? (heads ? TBL(cost_i8_heads) : TBL(cost_i8))
+                   : wt == ARIA_WF16 ? (heads ? TBL(cost_f16_heads) : TBL(cost_f16))
+                   : heads ? TBL(cost_q8_heads) : wt == ARIA_WQ4 ? TBL(cost_q4) : TBL(cost_q8);
+#undef TBL
+    const float k = (float)K / 1024.0f;
+    auto us = [&](const TileCost &c) {
+        const long T = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        return c.c0 + (float)((T + 255) / 256) * (c.c1 + c.ck * k);
+    };
+    /* fp16 HEADS runs on the LDS-operand kernel otherwise: 13.4 us at N = 1024 up to M = 1836, 14 -> 31 us
+     * at N = 3072 from M = 600 to 2592 */
+    float cur_us = wt == ARIA_WF16 && heads ? k * (12.0f + 2.5e-6f * (float)M * (float)N) : 1e30f;
+    for (int i = 0; i < tb.n; i++)
+        if (tb.t[i].pick == cur) cur_us = us(tb.t[i]);
+    int best = cur;
+    float best_us = 0.95f * cur_us;
+    const int steps = K / (wt == ARIA_WI8 ? 128 : 64);
+    for (int i = 0; i < tb.n; i++) {
+        const TileCost &c = tb.t[i];
+        /* only the K-split kernel and the large-tile configurations whose K is unsplit or even */
+        const bool split = c.pick < GEMM_KS && (wt == ARIA_WI8 ? c.pick == 4 || c.pick == 5 : wt != ARIA_WF16 && (c.pick == 5 || c.pick == 6));
+        if ((split && steps % 2) || (wt == ARIA_WF16 && c.pick < GEMM_KS)) continue;
+        const float t = us(c);
+        if (t < best_us) { best_us = t; best = c.pick; }
+    }
+    return best;
+}
+
 template <int WT, bool AF16>
 static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
     const bool aligned = a.K % BK == 0 && a.N % 4 == 0 && ((uintptr_t)a.x & 15u) == 0 &&
@@ -399,18 +465,22 @@ static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
         launch_cfg<C2, WT, AF16>(a, s);
         return hipGetLastError();
     } else {
+    if (tiles >= GEMM_KS) return qgemm_ks_launch(a, WT, tiles - GEMM_KS, s);   /* explicit: configuration tiles - GEMM_KS */
     if constexpr (WT == ARIA_WF16) {
         /* fp16 weights on the LDS-DMA kernel: explicit tiles 13.., or the configuration that
          * qgemm_big_f16_pick chooses for the shape (HEADS, which needs 64 columns per wave,
          * stays on the LDS-operand kernel) */
         if (tiles >= 13) return qgemm_big_launch(a, WT, tiles - 13, s);
-        if (tiles == 0 && a.K % 64 == 0 && (!a.gelu || a.epi.mode == ARIA_EPI_STORE) &&
-            a.epi.mode != ARIA_EPI_HEADS)
-            return qgemm_big_launch(a, WT, qgemm_big_f16_pick(a.M, a.N), s);
+        if (tiles == 0 && a.K % 64 == 0 && (!a.gelu || a.epi.mode == ARIA_EPI_STORE)) {
+            const bool heads = a.epi.mode == ARIA_EPI_HEADS;
+            const int c = qgemm_pick(WT, heads, a.M, a.N, a.K, heads ? -1 : qgemm_big_f16_pick(a.M, a.N));
+            if (c >= GEMM_KS) return qgemm_ks_launch(a, WT, c - GEMM_KS, s);
+            if (c >= 0) return qgemm_big_launch(a, WT, c, s);
+        }
     }
     if constexpr (WT != ARIA_WF16) {
         /* the LDS-DMA kernel (k_qgemm_big.hip): explicit tiles 13.. (configuration tiles - 13),
-         * or picked for the shapes where it measured fastest: N <= 1024 without HEADS (96 x 128
+         * or its configuration at M = 2592, from which qgemm_pick starts: N <= 1024 without HEADS (96 x 128
          * tiles, two workgroups per CU), HEADS with N <= 3072 (the qkv projection: 64 x 512 in
          * 8-wave workgroups, one per CU), other N <= 3072 without HEADS (128 x 128, two per CU), N = 4096
          * (192 x 256 in 8-wave workgroups, one per CU) and wider (224 x 128); N <= 1024 with an
@@ -426,7 +496,10 @@ static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
             const bool heads = a.epi.mode == ARIA_EPI_HEADS;
             const int cfg = heads ? (a.N <= 1024 && (a.K / 64) % 2 == 0 ? 6 : a.N <= 3072 ? 8 : -1)
                           : a.N <= 1024 ? ((a.K / 64) % 2 == 0 ? 5 : 0) : a.N <= 3072 ? 1 : a.N <= 4096 ? 7 : 4;
-            if (cfg >= 0) return qgemm_big_launch(a, WT, cfg, s);
+            if (cfg >= 0) {
+                const int c = qgemm_pick(WT, heads, a.M, a.N, a.K, cfg);
+                return c >= GEMM_KS ? qgemm_ks_launch(a, WT, c - GEMM_KS, s) : qgemm_big_launch(a, WT, c, s);
+            }
         }
         /* weights-in-registers kernel: explicit tiles 9..12 (BM = 32 * (tiles - 8)), or the pick */
         int fm = (tiles > NCFG) ? tiles - NCFG : (tiles == 0 ? pick_wr(a.M, a.N, a.K) : 0);

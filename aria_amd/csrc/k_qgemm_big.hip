@@ -35,8 +35,6 @@
 namespace {
 
 constexpr int KB = 64;   /* K-tile (fp16 activations) */
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x16_t __attribute__((ext_vector_type(16)));
 
 /* activation tile [BM][64] halves: 8 chunks of 16 B per row, logical chunk c of row r at
  * c ^ ((r >> 1) & 7) (conflict-free fragment reads: 32 rows x one chunk per lane half) */
@@ -48,28 +46,10 @@ struct WSt {              /* one lane's raw weights of one K-tile, FN 32-row blo
     uint32_t w[FN][NW];
 };
 
-__device__ __forceinline__ uint32_t and_or_v(uint32_t w, uint32_t mask, uint32_t magic) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(w), "s"(mask), "v"(magic));
-    return r;
-}
-
-/* the per-block offsets of the Q4 unpack: (1024 + n) * step + (min - 1024 step) = min + n step
- * for a low nibble, (1024 + 16 n) * step / 16 + (min - 64 step) for a high one */
-struct QOff { float a, b, st, s16; };
 template <int WT, int FN>
 __device__ __forceinline__ QOff qoff(const WSt<WT, FN> &s, int j) {
-    QOff o;
-    if constexpr (WT == ARIA_WQ4) {
-        const float mn = __builtin_bit_cast(float, s.w[j][4]);
-        o.st = __builtin_bit_cast(float, s.w[j][5]);
-        o.s16 = o.st * 0.0625f;
-        o.a = __builtin_fmaf(-1024.0f, o.st, mn);
-        o.b = __builtin_fmaf(-64.0f, o.st, mn);
-    } else {
-        o.a = o.b = o.st = o.s16 = 0.0f;
-    }
-    return o;
+    if constexpr (WT == ARIA_WQ4) return q4_off(__builtin_bit_cast(float, s.w[j][4]), __builtin_bit_cast(float, s.w[j][5]));
+    else return QOff{0.0f, 0.0f, 0.0f, 0.0f};
 }
 
 /* the 8 fp16 weights of block j for MFMA step ks (see k_qgemm_wr.hip for the arithmetic:
@@ -78,37 +58,12 @@ template <int WT, int FN>
 __device__ __forceinline__ half8_t wfrag(const WSt<WT, FN> &s, int j, int ks, uint32_t magic, const QOff &f) {
     uint32_t o[4];
     if constexpr (WT == ARIA_WQ4) {
-        const uint32_t w = s.w[j][ks], u = w >> 8;
-        const half2_t t0 = __builtin_bit_cast(half2_t, and_or_v(w, 0x000F000Fu, magic));
-        const half2_t t1 = __builtin_bit_cast(half2_t, and_or_v(w, 0x00F000F0u, magic));
-        const half2_t t2 = __builtin_bit_cast(half2_t, and_or_v(u, 0x000F000Fu, magic));
-        const half2_t t3 = __builtin_bit_cast(half2_t, and_or_v(u, 0x00F000F0u, magic));
-        const half2_t h0 = {(_Float16)__builtin_fmaf((float)t0[0], f.st, f.a), (_Float16)__builtin_fmaf((float)t1[0], f.s16, f.b)};
-        const half2_t h1 = {(_Float16)__builtin_fmaf((float)t2[0], f.st, f.a), (_Float16)__builtin_fmaf((float)t3[0], f.s16, f.b)};
-        const half2_t h2 = {(_Float16)__builtin_fmaf((float)t0[1], f.st, f.a), (_Float16)__builtin_fmaf((float)t1[1], f.s16, f.b)};
-        const half2_t h3 = {(_Float16)__builtin_fmaf((float)t2[1], f.st, f.a), (_Float16)__builtin_fmaf((float)t3[1], f.s16, f.b)};
-        o[0] = __builtin_bit_cast(uint32_t, h0); o[1] = __builtin_bit_cast(uint32_t, h1);
-        o[2] = __builtin_bit_cast(uint32_t, h2); o[3] = __builtin_bit_cast(uint32_t, h3);
+        return q4x8_to_h(s.w[j][ks], magic, f);
     } else {
         q8x4_to_h(s.w[j][2 * ks], o[0], o[1]);
         q8x4_to_h(s.w[j][2 * ks + 1], o[2], o[3]);
     }
     return __builtin_bit_cast(half8_t, make_uint4(o[0], o[1], o[2], o[3]));
-}
-
-/* s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding) */
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-/* One LDS DMA instruction: every lane moves 16 B from global address g to LDS byte address
- * m0 + 16 * lane (m0 wave-uniform). Issued as inline assembly, so the compiler neither waits
- * for it nor reorders memory accesses across it: the kernel waits on vmcnt itself. */
-__device__ __forceinline__ void dma16(const void *g, uint32_t m0) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(m0);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m), "v"(g) : "memory");
 }
 
 /* Layout of one pipeline stage in LDS (bytes):

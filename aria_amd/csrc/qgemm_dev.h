@@ -1,8 +1,8 @@
 /*
- * qgemm_dev.h - device code shared by the two dequant-on-use GEMM kernels
- * (k_qgemm.hip: both operands staged through LDS; k_qgemm_wr.hip: weights loaded
- * straight into registers): the kernel argument block, fp16 packing, the Q8 unpack,
- * the XCD-aware tile order and the fused epilogue. Included by those two files only.
+ * qgemm_dev.h - device code shared by the GEMM kernels (k_qgemm.hip: both operands staged
+ * through LDS; k_qgemm_wr.hip: weights loaded straight into registers; k_qgemm_big.hip: large
+ * tiles by LDS DMA; k_qgemm_ks.hip: small tiles, K split between waves; k_gemm_i8.hip): the
+ * kernel argument block, fp16 packing, the Q8 and Q4 unpack, LDS DMA and the fused epilogue.
  */
 #ifndef ARIA_QGEMM_DEV_H
 #define ARIA_QGEMM_DEV_H
@@ -28,6 +28,8 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x16_t __attribute__((ext_vector_type(16)));
 
 struct QArgs {
     void *y;
@@ -57,6 +59,51 @@ __device__ __forceinline__ void q8x4_to_h(uint32_t w, uint32_t &lo, uint32_t &hi
     const half2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
     lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - bias);
     hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - bias);
+}
+
+__device__ __forceinline__ uint32_t and_or_v(uint32_t w, uint32_t mask, uint32_t magic) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(w), "s"(mask), "v"(magic));
+    return r;
+}
+
+/* the per-block offsets of the Q4 unpack: (1024 + n) * step + (min - 1024 step) = min + n step
+ * for a low nibble, (1024 + 16 n) * step / 16 + (min - 64 step) for a high one */
+struct QOff { float a, b, st, s16; };
+__device__ __forceinline__ QOff q4_off(float mn, float st) {
+    return {__builtin_fmaf(-1024.0f, st, mn), __builtin_fmaf(-64.0f, st, mn), st, st * 0.0625f};
+}
+/* Q4: eight nibbles of one word (one quantization block) -> eight fp16 weights, each min + n step
+ * in fp32 (the value the reference dequantizes) rounded to fp16; magic = 0x64006400 in a VGPR */
+__device__ __forceinline__ half8_t q4x8_to_h(uint32_t w, uint32_t magic, const QOff &f) {
+    uint32_t o[4];
+    const uint32_t u = w >> 8;
+    const half2_t t0 = __builtin_bit_cast(half2_t, and_or_v(w, 0x000F000Fu, magic));
+    const half2_t t1 = __builtin_bit_cast(half2_t, and_or_v(w, 0x00F000F0u, magic));
+    const half2_t t2 = __builtin_bit_cast(half2_t, and_or_v(u, 0x000F000Fu, magic));
+    const half2_t t3 = __builtin_bit_cast(half2_t, and_or_v(u, 0x00F000F0u, magic));
+    const half2_t h0 = {(_Float16)__builtin_fmaf((float)t0[0], f.st, f.a), (_Float16)__builtin_fmaf((float)t1[0], f.s16, f.b)};
+    const half2_t h1 = {(_Float16)__builtin_fmaf((float)t2[0], f.st, f.a), (_Float16)__builtin_fmaf((float)t3[0], f.s16, f.b)};
+    const half2_t h2 = {(_Float16)__builtin_fmaf((float)t0[1], f.st, f.a), (_Float16)__builtin_fmaf((float)t1[1], f.s16, f.b)};
+    const half2_t h3 = {(_Float16)__builtin_fmaf((float)t2[1], f.st, f.a), (_Float16)__builtin_fmaf((float)t3[1], f.s16, f.b)};
+    o[0] = __builtin_bit_cast(uint32_t, h0); o[1] = __builtin_bit_cast(uint32_t, h1);
+    o[2] = __builtin_bit_cast(uint32_t, h2); o[3] = __builtin_bit_cast(uint32_t, h3);
+    return __builtin_bit_cast(half8_t, make_uint4(o[0], o[1], o[2], o[3]));
+}
+
+/* s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding) */
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+/* One LDS DMA instruction: every lane moves 16 B from global address g to LDS byte address
+ * m0 + 16 * lane (m0 wave-uniform). Issued as inline assembly, so the compiler neither waits
+ * for it nor reorders memory accesses across it: the kernel waits on vmcnt itself. */
+__device__ __forceinline__ void dma16(const void *g, uint32_t m0) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(m0);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m), "v"(g) : "memory");
 }
 
 /* xcd_tile (aria_dev.h) gives each XCD a contiguous run of tiles in M-major order, so an
@@ -423,5 +470,15 @@ int qgemm_big_f16_pick(int M, int N);
 /* its W8A8 form (int8 activations with per-row scales in a.xscale, Q8 weights, K % 128 == 0) */
 hipError_t qgemm_big_i8_launch(const QArgs &a, int cfg, hipStream_t s);
 int qgemm_big_i8_ncfg();
+
+/* the K-split kernel's launcher (k_qgemm_ks.hip): configuration cfg of qgemm_ks_ncfg(); wt is
+ * ARIA_WQ8, ARIA_WQ4, ARIA_WF16 (fp16 activations) or ARIA_WI8 (int8 ones), K % 64 == 0 */
+hipError_t qgemm_ks_launch(const QArgs &a, int wt, int cfg, hipStream_t s);
+int qgemm_ks_ncfg();
+/* the kernel for an M x N product of depth K: `cur` (a k_qgemm_big.hip configuration of this
+ * weight type, the pick at M = 2592) or another one of them, or GEMM_KS + a k_qgemm_ks.hip
+ * configuration (k_qgemm.hip) */
+#define GEMM_KS 100
+int qgemm_pick(int wt, bool heads, int M, int N, int K, int cur);
 
 #endif /* ARIA_QGEMM_DEV_H */
