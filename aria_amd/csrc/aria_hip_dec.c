@@ -6,8 +6,8 @@
  * create uploads the view once: the four block GEMM matrices, the 256 -> 768 projection as
  * fp16 (the reference's device decoder stores them so, src/aria_cuda.cu:1832-1880); the
  * ff_in rows and bias interleaved (value_i, gate_i) for the GEMM's GLU epilogue; the
- * folded mapping convolution [512, 768 * 3] as fp32, whose row layout already is the
- * im2col operand's; norms, biases, new tokens and the 34-position RoPE tables as fp32.
+ * folded mapping convolution [512, 768 * 3] as three bf16 parts per weight (24 bits, exact);
+ * norms, biases, new tokens and the 34-position RoPE tables as fp32.
  *
  * forward, latent [256, T] -> audio [2, T * 4096], one stream, every pass over all chunks:
  *   xt16 = half(latent * std)^T                        k_dec_in
@@ -24,8 +24,8 @@
  *     seq   += m16 . to_out^T; h16 = dyt(seq, ff_norm) k_qgemm (ADD_DYT epilogue)
  *     g16    = silu(gate) * value of h16 . ff_in^T + b k_qgemm (GLU epilogue)
  *     seq   += g16 . ff_out^T + b; h16 = dyt(seq, next pre_norm)  k_qgemm (ADD_DYT / ADD)
- *   xc   = im2col of the last 16 of each group          k_dec_im2col (first T * 16 rows)
- *   audio = unpatch(xc . mapping^T + b)                 k_dec_map (fp32 MFMA)
+ *   xs   = the last 16 of each group, split in bf16 parts  k_dec_split (first T * 16 rows)
+ *   audio = unpatch(conv(xs, mapping) + b)              k_dec_map (fp32 precision on the bf16 MFMA)
  * The workspace is kept on the handle and grown when a longer latent arrives.
  */
 #define __HIP_PLATFORM_AMD__ 1
@@ -58,7 +58,8 @@ typedef struct {
 struct aria_cuda_dec {
     float running_std;
     uint16_t *proj_w;
-    float *proj_b, *new_tokens, *mapping_w, *mapping_b, *rcos, *rsin;
+    void *mapping_w;   /* the split mapping weight (aria_k_dec_split_w) */
+    float *proj_b, *new_tokens, *mapping_b, *rcos, *rsin;
     dec_blk blk[6];
     hipStream_t st;
     void *ws;
@@ -93,6 +94,21 @@ static int up_f16(uint16_t **d, const float *h, size_t n, hipStream_t s) {
         hipError_t e = aria_k_f32_to_f16(*d, tmp, n, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) rc = aria_hip_fail(e, "decoder weight conversion");
+    }
+    if (tmp) hipFree(tmp);
+    return rc;
+}
+
+/* the folded mapping weight, fp32 host [512][768][3] -> its three bf16 parts on the device */
+static int up_split(void **d, const float *h, hipStream_t s) {
+    *d = NULL;
+    float *tmp = NULL;
+    int rc = up_f32(&tmp, h, (size_t)DOUT * 3 * DD);
+    if (!rc) rc = d_alloc(d, ARIA_DEC_WBYTES);
+    if (!rc) {
+        hipError_t e = aria_k_dec_split_w(*d, tmp, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) rc = aria_hip_fail(e, "decoder mapping weight");
     }
     if (tmp) hipFree(tmp);
     return rc;
@@ -162,8 +178,8 @@ aria_cuda_dec *aria_cuda_dec_create(const aria_sa3_dec_view *v) {
     }
     size_t fr = 0, tot = 0;
     hipMemGetInfo(&fr, &tot);
-    /* weights: 6 blocks of (3840 + 768 + 4608 + 2304) x 768 fp16, the fp32 mapping, headroom */
-    const size_t need = (size_t)6 * 11520 * DD * 2 + (size_t)DOUT * 3 * DD * 4 + ((size_t)256 << 20);
+    /* weights: 6 blocks of (3840 + 768 + 4608 + 2304) x 768 fp16, the split mapping, headroom */
+    const size_t need = (size_t)6 * 11520 * DD * 2 + ARIA_DEC_WBYTES + ((size_t)256 << 20);
     if (need > fr) {
         aria_hip_set_error("aria_cuda_dec_create: the decoder does not fit in device memory");
         return NULL;
@@ -179,7 +195,7 @@ aria_cuda_dec *aria_cuda_dec_create(const aria_sa3_dec_view *v) {
     int rc = up_f16(&h->proj_w, v->proj_w, (size_t)DD * 256, h->st);
     if (!rc) rc = up_f32(&h->proj_b, v->proj_b, DD);
     if (!rc) rc = up_f32(&h->new_tokens, v->new_tokens, DD);
-    if (!rc) rc = up_f32(&h->mapping_w, v->mapping_w, (size_t)DOUT * 3 * DD);
+    if (!rc) rc = up_split(&h->mapping_w, v->mapping_w, h->st);
     if (!rc) rc = up_f32(&h->mapping_b, v->mapping_b, DOUT);
     for (int i = 0; i < 6 && !rc; i++) rc = blk_create(&h->blk[i], &v->blocks[i], h->st);
     if (!rc) {
@@ -207,12 +223,13 @@ aria_cuda_dec *aria_cuda_dec_create(const aria_sa3_dec_view *v) {
  *   lat   [256, T] f32        xt16 [T, 256] f16       x [T, 768] f32
  *   seq   [L + 34, 768] f32   (the sequence at row 17; halos at rows 0-16, L + 17 ..)
  *   h16   [L + 34, 768] f16   m16 [L + 34, 768] f16
- *   qkv   [L + 34, 3840] f32  (after the blocks: xc [T * 16, 2304] f32)
+ *   qkv   [L + 34, 3840] f32  (after the blocks: xs, T * 16 + 2 rows of 4608 bytes)
  *   g16   [L + 34, 2304] f16
  *   audio [2, T * 4096] f32
  * L = 17 * Tp, Tp = T rounded up to even. */
 typedef struct {
-    float *lat, *x, *seq, *qkv, *xc, *audio;
+    float *lat, *x, *seq, *qkv, *audio;
+    void *xs;
     uint16_t *xt16, *h16, *m16, *g16;
 } dec_ws;
 
@@ -233,7 +250,7 @@ static size_t ws_layout(int T, dec_ws *w, char *base) {
     CARVE(audio, float, Lt * 512 * 4);
 #undef CARVE
     if (w) {
-        w->xc = w->qkv;                   /* Lt * 2304 * 4 <= R * 3840 * 4 */
+        w->xs = w->qkv;                   /* (Lt + 2) * 4608 <= R * 3840 * 4 */
     }
     return off;
 }
@@ -329,8 +346,8 @@ static int dec_run(aria_cuda_dec *h, const dec_ws *w, float *audio, const float 
                         hipMemcpyDeviceToDevice, s), "hipMemcpyAsync (halo)");
     for (int i = 3; i < 6; i++)
         if ((rc = block(h, &h->blk[i], i < 5 ? &h->blk[i + 1] : NULL, w, w->seq, w->h16, L / DS + 1, s))) return rc;
-    STEP(aria_k_dec_im2col(w->xc, seq, Lt, Lout, s), "k_dec_im2col");
-    STEP(aria_k_dec_map(audio, w->xc, h->mapping_w, h->mapping_b, Lt, s), "k_dec_map (mapping + unpatch)");
+    STEP(aria_k_dec_split(w->xs, seq, Lt, Lout, s), "k_dec_split");
+    STEP(aria_k_dec_map(audio, w->xs, h->mapping_w, h->mapping_b, Lt, 0, s), "k_dec_map (mapping + unpatch)");
     return 0;
 }
 

@@ -209,15 +209,23 @@ hipError_t aria_k_conv1d(float *out, const float *in, const float *w, const floa
  *   dec_attn:   merged fp16 [nch * 34, 768] = the differential attention of each chunk from
  *               qkv [nch * 34, 3840] (q | k | v | qd | kd), whose q/k sections already carry
  *               the DynamicTanh norms and RoPE (the to_qkv GEMM's DYT_ROPE epilogue)
- *   dec_im2col: xc fp32 [Lt, 2304] = the k3 mapping convolution's input rows
- *   dec_map:    audio [2, M * 256] = unpatch(xc [M, 2304] . W [512, 2304]^T + b), fp32 MFMA */
+ *   dec_split:  xs [Lt + 2 rows of ARIA_DEC_XROW bytes] = the mapping convolution's features, each
+ *               value as three bf16 parts (layout at k_dec_map); dec_split_w the folded weight
+ *               [512][768][3] likewise, ARIA_DEC_WBYTES bytes
+ *   dec_map:    audio [2, M * 256] = unpatch(conv(xs, ws) + b) at fp32 precision on the bf16 MFMA;
+ *               form 1 .. 3 = 64 x 64 (K over two wave groups), 128 x 128, 192 x 128 tiles, 0 =
+ *               picked */
+#define ARIA_DEC_XROW 4608
+#define ARIA_DEC_WBYTES ((size_t)512 * 72 * 192)
 hipError_t aria_k_dec_in(uint16_t *xt, const float *lat, int T, float std, hipStream_t s);
 hipError_t aria_k_dec_expand(float *seq, const float *x, const float *tok, int T, int Tp, hipStream_t s);
 hipError_t aria_k_dec_dyt(uint16_t *y, const float *x, float alpha, const float *g, const float *b, int rows,
                           hipStream_t s);
 hipError_t aria_k_dec_attn(uint16_t *merged, const float *qkv, int nch, hipStream_t s);
-hipError_t aria_k_dec_im2col(float *xc, const float *seq, int Lt, int Lout, hipStream_t s);
-hipError_t aria_k_dec_map(float *audio, const float *xc, const float *W, const float *b, int M, hipStream_t s);
+hipError_t aria_k_dec_split(void *xs, const float *seq, int Lt, int Lout, hipStream_t s);
+hipError_t aria_k_dec_split_w(void *ws, const float *W, hipStream_t s);
+hipError_t aria_k_dec_map(float *audio, const void *xs, const void *ws, const float *b, int M, int form,
+                          hipStream_t s);
 
 #ifdef __cplusplus
 }

@@ -12,8 +12,9 @@
  *                 softmax(q k^T / 8) v products over the chunk's 34 tokens on the fp32 MFMA,
  *                 their difference, merged fp16 (the q/k DynamicTanh norms and RoPE, 32
  *                 rotated dims, are the to_qkv GEMM's DYT_ROPE epilogue)
- *   k_dec_im2col  the k = 3 mapping convolution's input rows (the last 16 of each group)
- *   k_dec_map     the mapping convolution as an fp32 GEMM on the fp32 MFMA (the reference
+ *   k_dec_split   the k = 3 mapping convolution's input rows (the last 16 of each group), every
+ *                 value split into three bf16 parts
+ *   k_dec_map     the mapping convolution at fp32 precision on the bf16 MFMA (the reference
  *                 keeps it fp32), trimmed to T * 16 rows and unpatched to stereo in its stores
  * Arithmetic follows the reference's order (built with -ffp-contract=off). tanh: block 0's pre
  * norm (k_dec_dyt) uses the device library's tanhf; the other 11 block norms (the ADD_DYT
@@ -21,8 +22,7 @@
  * tanh_fast (exp + rcp, a few 1e-7 absolute, before the fp16 rounding of the GEMM operand);
  * the softmax exponential is v_exp_f32 (~1 ulp).
  */
-#include "aria_dev.h"
-#include "aria_hip_kernels.h"
+#include "qgemm_dev.h"   /* dma16, wait_vm */
 
 #define DEC_D 768
 #define DEC_S 34
@@ -247,154 +247,233 @@ __global__ __launch_bounds__(64 * DA_WAVES) void k_dec_attn_mfma(DecAttnArgs a, 
     }
 }
 
-/* xc[t][3 i + k] = seq token of feature position t + k - 1 (zero outside [0, Lout)), for the
- * first Lt positions (the trimmed output needs no more); feature position p is seq row
- * (p / 16) * 17 + 1 + p % 16, the last 16 of each group (src/aria_sa3_dec.c:85-99). The row
- * layout is the folded mapping weight's [512][768][3], so the k = 3 convolution is one GEMM. */
-__global__ __launch_bounds__(256) void k_dec_im2col(float *xc, const float *seq, int Lt, int Lout) {
-    const size_t n = (size_t)Lt * 3 * DEC_D;
+/* ---- the mapping convolution on the bf16 matrix cores, at fp32 precision ----
+ * audio[n / 256][m * 256 + n % 256] = sum over taps j < 3, i < 768 of feat[m + j - 1][i] W[n][i][j]
+ * + b[n], m < M = T * 16, n < 512 (src/aria_sa3_dec.c:85-116: the k = 3 convolution over the last
+ * 16 rows of each 17-row group, the trim and aria_unpatch_stereo). Feature position p is seq row
+ * (p / 16) * 17 + 1 + p % 16.
+ * The reference keeps this product in fp32. The fp32 MFMA runs at a sixteenth of the bf16 rate
+ * and bound it (307 us of a 60 s decode, 52 % of that pipe's peak; the im2col before it another 35
+ * us), so every fp32 operand is split into three bf16 parts, x = x0 + x1 + x2, each the top eight
+ * bits of what the parts before it left: 24 bits in all, so the split is exact. x y is then the six
+ * products x_i y_j with i + j <= 2; the three left out are below 2^-23 of x y. x0 y0 has an
+ * accumulator of its own and the five small products another, which is added at the end, so the
+ * large sum is rounded 144 times (once per MFMA) where the fp32 MFMA rounded it 1152 times.
+ * A non-finite operand keeps its class: the parts after x0 are zero, and a sum whose large part is
+ * not finite is that part alone. Relative error against float64, T = 1 .. 646 and values scaled by
+ * 1e-4 .. 300: 2.1-3.0e-7 where the fp32 MFMA had 6.1-8.6e-7. Time, split included: T = 108 64 -> 37 us,
+ * T = 300 140 -> 87 us, T = 646 261 -> 144 us.
+ *
+ * Layout: a row of 32-k blocks, 192 bytes each: the three parts of the block's 32 values, 64 bytes
+ * a part. Features sit in rows 1 .. of xs (row 0 and the row past the end are the convolution's
+ * zeros), 24 blocks = 4608 bytes a row, and W's k index is 768 j + i: an output row's 72 blocks
+ * are then three consecutive feature rows, 13824 contiguous bytes, and the convolution is one
+ * product over overlapping rows with nothing gathered. */
+#define MAP_KB 72                   /* 32-k blocks of an output row (2304 k) */
+#define MAP_BB 192                  /* bytes of a block: 3 parts x 32 bf16 */
+#define MAP_XROW (24 * MAP_BB)      /* bytes of a feature row */
+#define MAP_N 512
+
+/* the three bf16 parts of x, as bits; the remainders are exact in fp32 */
+__device__ __forceinline__ void bf16x3(float x, uint32_t (&p)[3]) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    p[0] = u >> 16;
+    p[1] = p[2] = 0;
+    if ((u & 0x7F800000u) == 0x7F800000u) {
+        if (u & 0x007FFFFFu) p[0] |= 0x0040u;   /* a NaN stays one without its low bits */
+        return;
+    }
+    const float r = x - __builtin_bit_cast(float, u & 0xFFFF0000u);
+    const uint32_t v = __builtin_bit_cast(uint32_t, r);
+    p[1] = v >> 16;
+    p[2] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, v & 0xFFFF0000u)) >> 16;
+}
+
+/* eight values -> a 16-byte chunk of each part */
+__device__ __forceinline__ void bf16x3_store(uint8_t *d, const float (&f)[8]) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        uint32_t a[3], b[3];
+        bf16x3(f[2 * e], a);
+        bf16x3(f[2 * e + 1], b);
+#pragma unroll
+        for (int p = 0; p < 3; p++) w[p][e] = a[p] | (b[p] << 16);
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) *reinterpret_cast<uint4 *>(d + 64 * p) = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+
+/* the split features, rows 0 .. Lt + 1: row r = feature position r - 1, zero outside [0, Lout) */
+__global__ __launch_bounds__(256) void k_dec_split(uint8_t *xs, const float *seq, int Lt, int Lout) {
+    const size_t n = (size_t)(Lt + 2) * (DEC_D / 8);
     for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < n; idx += (size_t)gridDim.x * 256) {
-        const int t = (int)(idx / (3 * DEC_D)), j = (int)(idx % (3 * DEC_D)), i = j / 3, k = j % 3;
-        const int tt = t + k - 1;
-        xc[idx] = (tt >= 0 && tt < Lout) ? seq[(size_t)((tt / 16) * 17 + 1 + tt % 16) * DEC_D + i] : 0.0f;
+        const int r = (int)(idx / (DEC_D / 8)), c = (int)(idx % (DEC_D / 8)), t = r - 1;
+        float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (t >= 0 && t < Lout) {
+            const float4 *s = reinterpret_cast<const float4 *>(seq + (size_t)((t / 16) * 17 + 1 + t % 16) * DEC_D + 8 * c);
+            const float4 u = s[0], v = s[1];
+            f[0] = u.x; f[1] = u.y; f[2] = u.z; f[3] = u.w; f[4] = v.x; f[5] = v.y; f[6] = v.z; f[7] = v.w;
+        }
+        bf16x3_store(xs + (size_t)r * MAP_XROW + (c >> 2) * MAP_BB + (c & 3) * 16, f);
     }
 }
 
-/* ---- the mapping convolution as an fp32 GEMM on the fp32 MFMA, unpatch fused ----
- * audio[n / 256][m * 256 + n % 256] = sum_k xc[m][k] W[n][k] + b[n], m < M = T * 16, n < 512,
- * k < 2304 (src/aria_sa3_dec.c:100-116: the mapping GEMM, the trim and aria_unpatch_stereo).
- * v_mfma_f32_32x32x2_f32 keeps fp32 operands, as the reference keeps this GEMM in fp32.
- * 256 threads = 2 x 2 waves, each owning FM x FN blocks of 32 x 32 (tile 64 FM rows of xc by
- * 64 FN rows of W); k moves through LDS 32 at a time, double-buffered (one barrier per
- * slice), the next slice's global loads in flight during the current slice's MFMAs. KS = 2
- * doubles the workgroup: the second 256 threads take the second half of k on their own
- * buffers and hand their partial sums to the first (acc_first + acc_second). The
- * MFMA computes W xc^T, so a lane's accumulators hold 4 consecutive n of one m: 4
- * consecutive audio samples, one 16-byte store. Lane l of an MFMA supplies row l % 32 at
- * k = 16 (l / 32) + j of the slice, j = 0..15 (any fixed k order gives the dot product),
- * so each lane reads 16 consecutive floats of its row: four 16-byte LDS reads. Rows past
- * M re-read row M - 1 and are not stored. */
-#define MAP_K 2304
-#define MAP_N 512
-#define MAP_KT 32
-#define MAP_SA 36          /* LDS row stride (floats): 16-byte reads of 16 rows hit 64 distinct banks */
+/* the split weights [512][72 blocks] from the folded mapping weight [512][768][3] */
+__global__ __launch_bounds__(256) void k_dec_split_w(uint8_t *ws, const float *W) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;   /* 512 x 288 chunks of eight k */
+    if (idx >= MAP_N * 4 * MAP_KB) return;
+    const int row = idx / (4 * MAP_KB), c = idx % (4 * MAP_KB), tap = c / 96, i0 = (c % 96) * 8;
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) f[e] = W[(size_t)row * 3 * DEC_D + (size_t)(i0 + e) * 3 + tap];
+    bf16x3_store(ws + ((size_t)row * MAP_KB + (c >> 2)) * MAP_BB + (c & 3) * 16, f);
+}
 
 typedef float f32x16_dec __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8_dec __attribute__((ext_vector_type(8)));
 
-template <int FM, int FN, int KS>
-__global__ __launch_bounds__(256 * KS) void k_dec_map(float *audio, const float *xc, const float *W, const float *bias, int M) {
-    constexpr int BM = 64 * FM, BN = 64 * FN;
-    constexpr int LA = BM * MAP_KT / 4 / 256, LW = BN * MAP_KT / 4 / 256;   /* float4 loads per thread */
-    /* KS = 2: threads 256.. (waves 4-7) run the second half of k on their own buffers, and
-     * their partial sums join the first half's through LDS before the stores */
-    __shared__ __attribute__((aligned(16))) float As_all[KS][2][BM * MAP_SA];
-    __shared__ __attribute__((aligned(16))) float Ws_all[KS][2][BN * MAP_SA];
-    static_assert(MAP_K % (MAP_KT * KS) == 0, "the k halves are whole slices");
-    const int khalf = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+/* A workgroup of KG groups of WM x WN waves, each wave FM x FN blocks of 32 x 32, owns 32 FM WM
+ * rows by 32 FN WN columns; group g takes the k blocks g, g + KG, .. on stages of its own, and the groups'
+ * sums meet in LDS in group order. A K step is one block: it moves by LDS DMA into one of NST
+ * stages, NST - 1 steps ahead, and a barrier publishes it. Chunk c of part p of row r is stored at
+ * 192 r + 64 p + 16 (c ^ ((r >> 2) & 3)): 16 lanes' fragment reads (16 rows, one chunk) touch
+ * all 64 banks once; MFMA step s of lane half h takes chunk 2 h + s on both sides. */
+template <int FM, int FN, int WM, int WN, int KG>
+__global__ __launch_bounds__(64 * WM * WN * KG) void k_dec_map(float *audio, const uint8_t *xs, const uint8_t *ws,
+                                                               const float *bias, int M) {
+    constexpr int W = WM * WN, BM = 32 * FM * WM, BN = 32 * FN * WN, SB = (BM + BN) * MAP_BB;   /* bytes of a stage */
+    constexpr int NST = 160 * 1024 / (KG * SB) > 3 ? 3 : 160 * 1024 / (KG * SB);
+    constexpr int DM = (SB / 1024 + W - 1) / W;   /* transfers per wave and step (the last ones may repeat) */
+    constexpr int KT = MAP_KB / KG;
+    /* the next step's transfers go out one by one between the MFMAs: a wave that issues them all
+     * at once waits at the full queue while its SIMD's matrix core idles (128 x 128 tiles: 81 -> 74
+     * us a launch of one round). One block per wave has too few MFMAs to spread them over. */
+    constexpr bool SPREAD = FM * FN > 1;
+    static_assert(NST >= 2 && SB % 1024 == 0 && MAP_KB % KG == 0 && MAP_N % BN == 0, "whole transfers and steps");
+    static_assert(KG == 1 || NST * SB >= 64 * W * FM * FN * 16 * 4, "a group's sums fit its stages");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[KG * NST * SB];
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / (64 * W)));
+    const int tid = threadIdx.x % (64 * W), wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wm = wave / WN, wn = wave % WN, lr = lane & 31, lh = lane >> 5;
+    uint8_t *const own = smem + grp * (NST * SB);
+    const uint32_t obase = (uint32_t)(uintptr_t)own;
+    /* tiles in row order per XCD: the columns of one row panel share its features in one L2 */
+    constexpr int NT = MAP_N / BN;
+    const int T = (M + BM - 1) / BM * NT, t = xcd_tile(blockIdx.x, T);
+    if (t >= T) return;                     /* uniform per workgroup, before any barrier */
+    const int m0 = t / NT * BM, n0 = t % NT * BN;
 
-    const int ntile = MAP_N / BN;
-    const int m0 = (blockIdx.x / ntile) * BM, n0 = (blockIdx.x % ntile) * BN;
-    const int tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
-    const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lh = lane >> 5;
+    /* transfer i of this wave: 64 chunks of the stage, feature rows first, then weight rows; rows
+     * past M re-read the last one */
+    const uint8_t *src[DM];
+#pragma unroll
+    for (int i = 0; i < DM; i++) {
+        const int q = 64 * min(W * i + wave, SB / 1024 - 1) + lane, r = q / 12, p = q % 12, c = (p & 12) | ((p & 3) ^ ((r >> 2) & 3));
+        src[i] = r < BM ? xs + (size_t)min(m0 + r, M - 1) * MAP_XROW + 16 * c
+                        : ws + (size_t)(n0 + r - BM) * (MAP_KB * MAP_BB) + 16 * c;
+    }
+    auto issue1 = [&](int i, int st, int kt) __attribute__((always_inline)) {
+        dma16(src[i] + (size_t)(grp + KG * kt) * MAP_BB, obase + st * SB + 1024 * min(W * i + wave, SB / 1024 - 1));
+    };
+    auto issue = [&](int st, int kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < DM; i++) issue1(i, st, kt);
+    };
+    auto barrier = []() __attribute__((always_inline)) {   /* every fragment read has returned; transfers stay in flight */
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
 
-    f32x16_dec acc[FM][FN];
+    f32x16_dec hi[FM][FN], lo[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
         for (int j = 0; j < FN; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; r++) hi[i][j][r] = lo[i][j][r] = 0.0f;
 
-    auto compute = [&](int buf) {
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-            float4 xa[FM], wa[FN];
+    for (int p = 0; p < NST - 1; p++) issue(p, p);
+    wait_vm<(NST - 2) * DM>();
+    barrier();
+    int st = 0;
+    for (int kt = 0; kt < KT; kt++) {
+        const bool more = kt + NST - 1 < KT;
+        const int nst = st == 0 ? NST - 1 : st - 1;
+        if (!SPREAD && more) issue(nst, kt + NST - 1);
+        const uint8_t *S = own + st * SB;
+        bf16x8_dec x[2][3][FM], w[2][3][FN];   /* every read of the step is requested before its first MFMA */
 #pragma unroll
-            for (int i = 0; i < FM; i++)
-                xa[i] = *reinterpret_cast<const float4 *>(&As_all[khalf][buf][(wm * 32 * FM + i * 32 + lr) * MAP_SA + lh * 16 + q4 * 4]);
+        for (int s = 0; s < 2; s++) {
+            const int off = lr * MAP_BB + 16 * ((2 * lh + s) ^ ((lr >> 2) & 3));
 #pragma unroll
-            for (int j = 0; j < FN; j++)
-                wa[j] = *reinterpret_cast<const float4 *>(&Ws_all[khalf][buf][(wn * 32 * FN + j * 32 + lr) * MAP_SA + lh * 16 + q4 * 4]);
+            for (int p = 0; p < 3; p++) {
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+                for (int i = 0; i < FM; i++)
+                    x[s][p][i] = *reinterpret_cast<const bf16x8_dec *>(S + (wm * 32 * FM + 32 * i) * MAP_BB + off + 64 * p);
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    w[s][p][j] = *reinterpret_cast<const bf16x8_dec *>(S + (BM + wn * 32 * FN + 32 * j) * MAP_BB + off + 64 * p);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int q = 0; q < 6; q++) {   /* in the order in which the operands arrive */
+                constexpr int pw[6] = {0, 0, 1, 1, 0, 2}, px[6] = {0, 1, 0, 1, 2, 0};
 #pragma unroll
                 for (int i = 0; i < FM; i++)
 #pragma unroll
-                    for (int j = 0; j < FN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[j][e], xa[i][e], acc[i][j], 0, 0, 0);
-        }
-    };
-
-    /* per thread: float4 q = tid + 256 i of the slice, row q / 8, column 4 (q % 8) */
-    const float *ga[LA], *gw[LW];
-    constexpr int NK = MAP_K / MAP_KT / KS;   /* slices of this half */
-    const int k0 = khalf * NK * MAP_KT;
+                    for (int j = 0; j < FN; j++) {
+                        if (q == 0) hi[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s][0][j], x[s][0][i], hi[i][j], 0, 0, 0);
+                        else lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s][pw[q]][j], x[s][px[q]][i], lo[i][j], 0, 0, 0);
+                    }
+                if constexpr (SPREAD) {
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < LA; i++) {
-        const int q = tid + i * 256;
-        ga[i] = xc + (size_t)min(m0 + (q >> 3), M - 1) * MAP_K + k0 + (q & 7) * 4;
+                    for (int i = 6 * s + q; i < DM; i += 12)
+                        if (more) issue1(i, nst, kt + NST - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        if (more) wait_vm<(NST - 2) * DM>();
+        else wait_vm<0>();
+        barrier();
+        st = st + 1 == NST ? 0 : st + 1;
     }
 #pragma unroll
-    for (int i = 0; i < LW; i++) {
-        const int q = tid + i * 256;
-        gw[i] = W + (size_t)(n0 + (q >> 3)) * MAP_K + k0 + (q & 7) * 4;
-    }
-    const int so = (tid >> 3) * MAP_SA + (tid & 7) * 4;   /* + 32 rows per i */
-    float4 ra[LA], rw[LW];
+    for (int i = 0; i < FM; i++)
 #pragma unroll
-    for (int i = 0; i < LA; i++) ra[i] = *reinterpret_cast<const float4 *>(ga[i]);
+        for (int j = 0; j < FN; j++)
 #pragma unroll
-    for (int i = 0; i < LW; i++) rw[i] = *reinterpret_cast<const float4 *>(gw[i]);
-#pragma unroll
-    for (int i = 0; i < LA; i++) *reinterpret_cast<float4 *>(&As_all[khalf][0][so + i * 32 * MAP_SA]) = ra[i];
-#pragma unroll
-    for (int i = 0; i < LW; i++) *reinterpret_cast<float4 *>(&Ws_all[khalf][0][so + i * 32 * MAP_SA]) = rw[i];
-    __syncthreads();
-    for (int kt = 0; kt < NK; kt++) {
-        const int cur = kt & 1;
-        if (kt + 1 < NK) {
-#pragma unroll
-            for (int i = 0; i < LA; i++) ra[i] = *reinterpret_cast<const float4 *>(ga[i] + (kt + 1) * MAP_KT);
-#pragma unroll
-            for (int i = 0; i < LW; i++) rw[i] = *reinterpret_cast<const float4 *>(gw[i] + (kt + 1) * MAP_KT);
-        }
-        compute(cur);
-        if (kt + 1 < NK) {
-#pragma unroll
-            for (int i = 0; i < LA; i++) *reinterpret_cast<float4 *>(&As_all[khalf][cur ^ 1][so + i * 32 * MAP_SA]) = ra[i];
-#pragma unroll
-            for (int i = 0; i < LW; i++) *reinterpret_cast<float4 *>(&Ws_all[khalf][cur ^ 1][so + i * 32 * MAP_SA]) = rw[i];
-        }
-        __syncthreads();
-    }
-
-    if constexpr (KS == 2) {
-        /* every wave is past its last LDS read (the loop's closing barrier): the second half's
-         * partial sums go through its own buffers, lane-major, and the first half adds them
-         * (acc_first + acc_second, a fixed order) and stores */
-        float *X = &As_all[1][0][0] + tid;
-        static_assert(FM * FN * 16 * 256 <= 2 * BM * MAP_SA, "the partial sums fit the second half's buffers");
-        if (khalf == 1) {
+            for (int r = 0; r < 16; r++) {
+                const float h = hi[i][j][r];
+                hi[i][j][r] = __builtin_isfinite(h) ? h + lo[i][j][r] : h;
+            }
+    if constexpr (KG == 2) {
+        float *X = reinterpret_cast<float *>(smem + NST * SB) + tid;   /* the second group's stages, lane-major */
+        if (grp == 1) {
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
                 for (int j = 0; j < FN; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) X[((i * FN + j) * 16 + r) * 256] = acc[i][j][r];
+                    for (int r = 0; r < 16; r++) X[((i * FN + j) * 16 + r) * 64 * W] = hi[i][j][r];
         }
         __syncthreads();
-        if (khalf == 0) {
+        if (grp == 1) return;
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+        for (int i = 0; i < FM; i++)
 #pragma unroll
-                for (int j = 0; j < FN; j++)
+            for (int j = 0; j < FN; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) acc[i][j][r] = acc[i][j][r] + X[((i * FN + j) * 16 + r) * 256];
-        }
+                for (int r = 0; r < 16; r++) hi[i][j][r] = hi[i][j][r] + X[((i * FN + j) * 16 + r) * 64 * W];
     }
-    if (KS == 2 && khalf == 1) return;
-
-    /* accumulator r of lane l: n = 8 (r / 4) + 4 (l / 32) + r % 4, m = l % 32 (per block) */
+    /* accumulator r of lane l: n = 8 (r / 4) + 4 (l / 32) + r % 4, m = l % 32 (per block): 4
+     * consecutive audio samples per 16-byte store */
 #pragma unroll
     for (int i = 0; i < FM; i++) {
         const int m = m0 + wm * 32 * FM + i * 32 + lr;
@@ -405,12 +484,9 @@ __global__ __launch_bounds__(256 * KS) void k_dec_map(float *audio, const float 
             for (int g = 0; g < 4; g++) {
                 const int n = n0 + wn * 32 * FN + j * 32 + 8 * g + 4 * lh;
                 const float4 b = *reinterpret_cast<const float4 *>(bias + n);
-                float4 o;
-                o.x = acc[i][j][4 * g + 0] + b.x;
-                o.y = acc[i][j][4 * g + 1] + b.y;
-                o.z = acc[i][j][4 * g + 2] + b.z;
-                o.w = acc[i][j][4 * g + 3] + b.w;
-                *reinterpret_cast<float4 *>(audio + (size_t)(n >> 8) * M * 256 + (size_t)m * 256 + (n & 255)) = o;
+                *reinterpret_cast<float4 *>(audio + (size_t)(n >> 8) * M * 256 + (size_t)m * 256 + (n & 255)) =
+                    make_float4(hi[i][j][4 * g] + b.x, hi[i][j][4 * g + 1] + b.y, hi[i][j][4 * g + 2] + b.z,
+                                hi[i][j][4 * g + 3] + b.w);
             }
     }
 }
@@ -445,23 +521,38 @@ extern "C" hipError_t aria_k_dec_attn(uint16_t *merged, const float *qkv, int nc
     hipLaunchKernelGGL(k_dec_attn_mfma, dim3(nch * 12), dim3(64 * DA_WAVES), 0, s, a, 12);
     return hipGetLastError();
 }
-extern "C" hipError_t aria_k_dec_im2col(float *xc, const float *seq, int Lt, int Lout, hipStream_t s) {
-    hipLaunchKernelGGL(k_dec_im2col, grid_for((size_t)Lt * 3 * DEC_D), dim3(256), 0, s, xc, seq, Lt, Lout);
+extern "C" hipError_t aria_k_dec_split(void *xs, const float *seq, int Lt, int Lout, hipStream_t s) {
+    hipLaunchKernelGGL(k_dec_split, grid_for((size_t)(Lt + 2) * (DEC_D / 8)), dim3(256), 0, s, (uint8_t *)xs, seq, Lt, Lout);
     return hipGetLastError();
 }
-/* audio [2, M * 256] = unpatch(xc [M, 2304] . W [512, 2304]^T + b) in 64 x 64 tiles: faster
- * than 128 x 64, 64 x 128 and 128 x 128 at every decoder length measured (T = 108, 646, 2584;
- * every tiling gives the same bits) */
-extern "C" hipError_t aria_k_dec_map(float *audio, const float *xc, const float *W, const float *b, int M,
+extern "C" hipError_t aria_k_dec_split_w(void *ws, const float *W, hipStream_t s) {
+    hipLaunchKernelGGL(k_dec_split_w, dim3(MAP_N * 4 * MAP_KB / 256), dim3(256), 0, s, (uint8_t *)ws, W);
+    return hipGetLastError();
+}
+template <int FM, int FN, int WM, int WN, int KG>
+static void launch_map(float *audio, const void *xs, const void *ws, const float *b, int M, hipStream_t s) {
+    const int T = (M + 32 * FM * WM - 1) / (32 * FM * WM) * (MAP_N / (32 * FN * WN));
+    hipLaunchKernelGGL((k_dec_map<FM, FN, WM, WN, KG>), dim3((T + 7) / 8 * 8), dim3(64 * WM * WN * KG), 0, s, audio,
+                       (const uint8_t *)xs, (const uint8_t *)ws, b, M);
+}
+extern "C" hipError_t aria_k_dec_map(float *audio, const void *xs, const void *ws, const float *b, int M, int form,
                                      hipStream_t s) {
     if (M <= 0) return hipSuccess;
-    /* at most one tile per CU (T <= 128: 216 tiles at T = 108): the k range split over two
-     * 4-wave halves gives each SIMD two waves (decode 0.688 -> 0.658 ms at T = 108); more tiles
-     * keep one 4-wave workgroup per tile (the split measured 0.5 % slower at T = 646) */
-    const int tiles = (M + 63) / 64 * (MAP_N / 64);
-    if (tiles <= 256)
-        hipLaunchKernelGGL((k_dec_map<1, 1, 2>), dim3(tiles), dim3(512), 0, s, audio, xc, W, b, M);
-    else
-        hipLaunchKernelGGL((k_dec_map<1, 1, 1>), dim3(tiles), dim3(256), 0, s, audio, xc, W, b, M);
+    if (form == 0) {
+        /* the fewest us of the busiest CU: tiles of 64 x 64 with K over two wave groups take 30 us
+         * (216 tiles at T = 108: 34 us), 128 x 128 80 us (T = 300: 81 us; the 64 x 64 form 92 us), 192 x
+         * 128 122 us (T = 646, 216 tiles: 131 us; 128 x 128 in two rounds 170 us) */
+        const int mt[3] = {(M + 63) / 64 * 8, (M + 127) / 128 * 4, (M + 191) / 192 * 4};
+        const int us[3] = {30, 80, 122};
+        int best = 1 << 30;
+        for (int i = 0; i < 3; i++) {
+            const int c = (mt[i] + 255) / 256 * us[i];
+            if (c < best) { best = c; form = i + 1; }
+        }
+    }
+    if (form == 1) launch_map<1, 1, 2, 2, 2>(audio, xs, ws, b, M, s);
+    else if (form == 2) launch_map<2, 2, 2, 2, 1>(audio, xs, ws, b, M, s);
+    else if (form == 3) launch_map<3, 2, 2, 2, 1>(audio, xs, ws, b, M, s);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
