@@ -386,7 +386,7 @@ static int pick_wr(int M, int N, int K) {
  * M = 40 .. 2592 over the DiT's projections (N / K = 1024 / 1024, 3072 / 1024, 4096 / 1024,
  * 8192 / 1024, 1024 / 4096), each launch alone in a replayed graph over six operand sets; rms
  * error 5-9 %. A candidate displaces the configuration that M = 2592 takes only where it is
- * predicted 5 % faster. Over the sweep the picks run 1.64x (Q8, Q4), 1.24x (fp16), 1.52x (int8),
+ * predicted 8 % faster. Over the sweep the picks run 1.64x (Q8, Q4), 1.24x (fp16), 1.52x (int8),
  * HEADS 1.6-1.9x faster than those configurations in the geometric mean and are within 1-2 % of
  * the fastest of each shape on average (fp16 4 %). Down to two rows of tiles the small tiles of
  * k_qgemm_ks.hip win because they give every CU work; from about M = 860 (N = 8192) to 1420
@@ -405,7 +405,7 @@ static const TileCost cost_f16[] = {{GEMM_KS, 32, 32, 1.1f, 1.6f, 1.5f}, {GEMM_K
     {2, 128, 128, 5.0f, 1.0f, 9.9f}, {3, 160, 128, 6.1f, 0.7f, 11.2f}, {4, 192, 128, 6.8f, 1.6f, 12.0f}};
 static const TileCost cost_i8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 0.8f}, {GEMM_KS + 1, 32, 64, 0.9f, 2.2f, 1.1f},
     {GEMM_KS + 2, 64, 64, 0.9f, 3.4f, 1.4f}, {GEMM_KS + 3, 96, 64, 1.4f, 4.1f, 1.9f}, {0, 64, 128, 2.0f, 3.1f, 2.2f},
-    {2, 128, 128, 5.1f, 1.3f, 4.9f}, {3, 192, 128, 6.6f, 2.3f, 5.7f}, {4, 96, 128, -0.2f, 6.1f, 3.4f},
+    {2, 128, 128, 6.0f, 0.2f, 4.9f}, {3, 192, 128, 7.5f, 2.3f, 5.7f}, {4, 96, 128, -0.2f, 6.1f, 3.4f},
     {6, 192, 256, -6.7f, 12.3f, 12.3f}};
 /* HEADS (64 columns in one wave; timed at K = 1024 only, N = 1024 and 3072) */
 static const TileCost cost_q8_heads[] = {{GEMM_KS + 1, 32, 64, 1.1f, 2.4f, 2.0f}, {GEMM_KS + 3, 96, 64, 2.0f, 5.4f, 3.2f},
@@ -434,7 +434,7 @@ int qgemm_pick(int wt, bool heads, int M, int N, int K, int cur) {
     for (int i = 0; i < tb.n; i++)
         if (tb.t[i].pick == cur) cur_us = us(tb.t[i]);
     int best = cur;
-    float best_us = 0.95f * cur_us;
+    float best_us = 0.92f * cur_us;
     const int steps = K / (wt == ARIA_WI8 ? 128 : 64);
     for (int i = 0; i < tb.n; i++) {
         const TileCost &c = tb.t[i];
