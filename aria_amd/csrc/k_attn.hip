@@ -210,29 +210,30 @@ __device__ __forceinline__ uint32_t pack2h_rn(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2_v));
 }
 
-/* QW (3 to 6) waves of 32 queries per key half. KS = 1: all keys. KS = 2: 2 QW waves; waves QW..2 QW - 1
+/* QW (3 to 6; KS = 4: 1 or 2) waves of 32 queries per key slice. KS = 1: all keys. KS = 2: 2 QW waves; waves QW..2 QW - 1
  * take the second half of the key tiles with their own LDS buffers, and the halves merge
  * (max, row sum, O) through LDS at the end: twice the waves per query block without any
- * exchange between workgroups. Both halves run the same number of loop trips, so every
- * barrier is reached by all waves. */
-template <int KS, int QW>
-__global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(4))) void k_flash_attn(AttnArgs a) {
+ * exchange between workgroups. KS = 4: four slices likewise, merged by all waves. Every slice
+ * runs the same number of loop trips, so every barrier is reached by all waves. */
+template <int KS, int QW, bool ONE = false>
+__global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS > 2 ? 2 : 4))) void k_flash_attn(AttnArgs a) {
     /* tile buffers, each [half][KT x 64] fp16, as four separate LDS objects: K and V tiles
      * arrive by LDS DMA (global_load_lds), whose writes count on vmcnt, and the compiler only
      * omits a vmcnt wait before a fragment read when the read provably targets another object
      * than the pending DMA. After the key loop Kb0s + Kb1s hold the merge exchange (4 waves x
      * 34 x 64 floats = 34.8 KB; the two objects are placed back to back, checked below). */
+    constexpr int SECOND = ONE ? 64 : KS * KT * 64;   /* ONE: a slice's keys are one tile */
     __shared__ __attribute__((aligned(16))) uint16_t Kb0s[KS * KT * 64];
-    __shared__ __attribute__((aligned(16))) uint16_t Kb1s[KS * KT * 64];
+    __shared__ __attribute__((aligned(16))) uint16_t Kb1s[SECOND];
     __shared__ __attribute__((aligned(16))) uint16_t Vb0s[KS * KT * 64];
-    __shared__ __attribute__((aligned(16))) uint16_t Vb1s[KS * KT * 64];
+    __shared__ __attribute__((aligned(16))) uint16_t Vb1s[SECOND];
 
-    static_assert(QW >= 3 && QW <= 6, "three to six query waves per key half");
+    static_assert(KS > 2 ? QW <= 2 && 8 % KS == 0 : !ONE && QW >= 3 && QW <= 6, "query waves per key slice");
     /* the wave index in a scalar register: everything derived from it stays scalar */
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int half = KS == 1 ? 0 : wid / QW;
-    uint16_t *const Kb0 = Kb0s + half * (KT * 64), *const Kb1 = Kb1s + half * (KT * 64);
-    uint16_t *const Vb0 = Vb0s + half * (KT * 64), *const Vb1 = Vb1s + half * (KT * 64);
+    uint16_t *const Kb0 = Kb0s + half * (KT * 64), *const Kb1 = Kb1s + (ONE ? 0 : half * (KT * 64));
+    uint16_t *const Vb0 = Vb0s + half * (KT * 64), *const Vb1 = Vb1s + (ONE ? 0 : half * (KT * 64));
     const int lane = threadIdx.x & 63, wave = wid % QW, g = lane >> 5, l32 = lane & 31;
     if ((int)blockIdx.x >= a.Tpad) {        /* a prefetch workgroup (uniform, before any barrier) */
         attn_prefetch(a, (int)blockIdx.x - a.Tpad, (int)gridDim.x - a.Tpad);
@@ -399,6 +400,10 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(4)
      * past Nq (in the last query block: 1296 = 6 x 192 + 144, so that block's sixth wave)
      * only stages tiles and meets the barriers; its products would never be stored. */
     const bool live = q0 < a.Nq;
+    if constexpr (ONE) {   /* niter is 1 (the launcher's choice) */
+        if (live && nt > 0) tile(kbase, K0, V0);
+        __syncthreads();
+    } else
     for (int t = 0; t < niter; t += 2) {
         if (t + 1 < nt) dma(kbase + (t + 1) * KT, Kb1, Vb1);
         if (live && t < nt) tile(kbase + t * KT, K0, V0);
@@ -414,6 +419,58 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(4)
 
     float lrow = lsum + xor32_f32(lsum, lane);   /* the query's full row sum */
 
+    if constexpr (KS > 2) {
+        /* merge: every slice leaves its O (eight groups of four registers: dims 32 dt + 8 rq + 4 g ..
+         * of the lane's query), l and m in LDS (the tile buffers are free after the last trip's
+         * barrier), and slice h finishes 8 / KS of the groups of its query wave. A slice without
+         * keys has m = -inf and l = O = 0: weight zero (slice 0 always has keys). */
+        __shared__ __attribute__((aligned(16))) float lm[2 * KS * QW * 64];
+        static_assert(KS * KT * 64 * 2 >= KS * QW * 4 * 64 * 16, "the O groups fit the tile buffers");
+        float4 *const x0 = reinterpret_cast<float4 *>(Kb0s), *const x1 = reinterpret_cast<float4 *>(Vb0s);
+        const int slot = half * QW + wave;
+#pragma unroll
+        for (int rq = 0; rq < 4; rq++) {
+            x0[(slot * 4 + rq) * 64 + lane] = make_float4(oacc[0][4 * rq], oacc[0][4 * rq + 1], oacc[0][4 * rq + 2], oacc[0][4 * rq + 3]);
+            x1[(slot * 4 + rq) * 64 + lane] = make_float4(oacc[1][4 * rq], oacc[1][4 * rq + 1], oacc[1][4 * rq + 2], oacc[1][4 * rq + 3]);
+        }
+        lm[slot * 64 + lane] = lrow;
+        lm[(KS * QW + slot) * 64 + lane] = m_use;
+        __syncthreads();
+        float w[KS], m = -INFINITY, l = 0.0f;
+#pragma unroll
+        for (int h = 0; h < KS; h++) {
+            w[h] = lm[(KS * QW + h * QW + wave) * 64 + lane];
+            m = fmaxf(m, w[h]);
+        }
+#pragma unroll
+        for (int h = 0; h < KS; h++) {
+            w[h] = __builtin_amdgcn_exp2f(w[h] - m);
+            l += lm[(h * QW + wave) * 64 + lane] * w[h];
+        }
+        const int qi = q0 + l32;
+        if (qi >= a.Nq) return;
+        const float inv = 1.0f / l;
+        const size_t orow = ((size_t)(bh / a.H) * a.Nq + qi) * (size_t)(a.H * 64) + (bh % a.H) * 64;
+#pragma unroll
+        for (int i = 0; i < 8 / KS; i++) {
+            const int gr = half * (8 / KS) + i, rq = gr & 3;
+            const float4 *x = gr < 4 ? x0 : x1;
+            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int h = 0; h < KS; h++) {
+                const float4 v = x[((h * QW + wave) * 4 + rq) * 64 + lane];
+                o = make_float4(o.x + v.x * w[h], o.y + v.y * w[h], o.z + v.z * w[h], o.w + v.w * w[h]);
+            }
+            const int d = 32 * (gr >> 2) + 8 * rq + 4 * g;
+            if (a.o_f16)
+                *reinterpret_cast<uint2 *>((uint16_t *)a.o + orow + d) =
+                    make_uint2(pack2h_rn(o.x * inv, o.y * inv), pack2h_rn(o.z * inv, o.w * inv));
+            else
+                *reinterpret_cast<float4 *>((float *)a.o + orow + d) =
+                    make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+        }
+        return;
+    }
     if constexpr (KS == 2) {
         /* merge: the second half hands (O, l, m) to the first through LDS (the tile buffers
          * are free after the last trip's barrier): per wave 64 lanes x 16 floats of each O
@@ -493,9 +550,21 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
      * queries (31.9 -> 27.8 us against 352 blocks of 128; the same bits). The one-half form
      * takes the fewest query slots on the busiest CU (ceil(T / 256) blocks of 32 QW queries),
      * ties to 4: the cross attention at S = 1296, 32 heads takes 3 (10.8 -> 10.4 us) */
-    const bool split = (Nk + KT - 1) / KT >= 8;
+    const int tiles = (Nk + KT - 1) / KT;
+    const bool split = tiles >= 8;
+    /* few queries: the keys in four slices, with one or two query waves each, while that leaves
+     * every CU at most one workgroup. A workgroup then walks a quarter of the key tiles and
+     * twice to four times as many CUs work: one sequence of 172 (16 heads, 3 tiles) 5.9 -> 4.6 us,
+     * 172 x 256 keys 6.3 -> 4.4, 344 8.3 -> 6.0, two of 512 9.6 -> 7.9, 710 11.6 -> 9.2, 1000 14.7 -> 10.9.
+     * Past one workgroup per CU it loses (1296: 17.6 -> 23.6 us), as it does with too few tiles to
+     * share (40 keys 4.0 -> 4.3; two query waves on 100 keys 5.2 -> 5.5). Eight slices of one wave
+     * were slower than four at every length up to 512 keys. */
+    const long t1 = (long)((Nq + 31) / 32) * BH, t2 = (long)((Nq + 63) / 64) * BH;
+    const int four = tiles >= 2 && t1 <= 256 ? 1 : tiles >= 3 && t2 <= 256 ? 2 : 0;
     int qw = 4;
-    if (split) {
+    if (four) {
+        qw = four;
+    } else if (split) {
         for (int w = 4; w <= 6; w++)
             if ((long)((Nq + 32 * w - 1) / (32 * w)) * BH <= 256) { qw = w; break; }
     } else {
@@ -512,10 +581,16 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
         ncu = (hipGetDevice(&dev) == hipSuccess &&
                hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : -1;
     }
-    const int npw = (split && a.npf && ncu > a.Tpad) ? (ncu - a.Tpad) / 8 * 8 : 0;
+    const int npw = (split && !four && a.npf && ncu > a.Tpad) ? (ncu - a.Tpad) / 8 * 8 : 0;
     if (!npw) a.npf = 0;
     const dim3 grid(a.Tpad + npw);
-    if (split) {
+    if (four) {
+        const bool one = tiles <= 4;   /* a tile per slice: no second buffers */
+        if (four == 1 && one) hipLaunchKernelGGL((k_flash_attn<4, 1, true>), grid, dim3(256), 0, s, a);
+        else if (four == 1) hipLaunchKernelGGL((k_flash_attn<4, 1>), grid, dim3(256), 0, s, a);
+        else if (one) hipLaunchKernelGGL((k_flash_attn<4, 2, true>), grid, dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((k_flash_attn<4, 2>), grid, dim3(512), 0, s, a);
+    } else if (split) {
         if (qw == 6) hipLaunchKernelGGL((k_flash_attn<2, 6>), grid, dim3(768), 0, s, a);
         else if (qw == 5) hipLaunchKernelGGL((k_flash_attn<2, 5>), grid, dim3(640), 0, s, a);
         else hipLaunchKernelGGL((k_flash_attn<2, 4>), grid, dim3(512), 0, s, a);
