@@ -289,7 +289,10 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
     float lsum = 0.0f;
     typedef _Float16 half2_v __attribute__((ext_vector_type(2)));
     const half2_v one2 = {(_Float16)1.0f, (_Float16)1.0f};
-    float m_use = -INFINITY;   /* running reference max, scaled (log2) units */
+    /* running reference max, scaled (log2) units. Four slices start it finite, below every finite
+     * score (fp16 operands: |s| < 1e11): a slice whose keys all score -inf then has l = O = 0 (not
+     * exp2 of -inf + inf) and weight zero against the others. Every score -inf gives 0 / 0 */
+    float m_use = KS > 2 ? -3e38f : -INFINITY;
 
     /* per-lane LDS offsets (halves) of the fragment reads, hoisted out of the key loop. The
      * swizzles depend only on lane bits: K block kb (keys 32kb..) sits 32*64*kb further, V key
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
         /* merge: every slice leaves its O (eight groups of four registers: dims 32 dt + 8 rq + 4 g ..
          * of the lane's query), l and m in LDS (the tile buffers are free after the last trip's
          * barrier), and slice h finishes 8 / KS of the groups of its query wave. A slice without
-         * keys has m = -inf and l = O = 0: weight zero (slice 0 always has keys). */
+         * keys has the starting m and l = O = 0: weight zero (slice 0 always has keys). */
         __shared__ __attribute__((aligned(16))) float lm[2 * KS * QW * 64];
         static_assert(KS * KT * 64 * 2 >= KS * QW * 4 * 64 * 16, "the O groups fit the tile buffers");
         float4 *const x0 = reinterpret_cast<float4 *>(Kb0s), *const x1 = reinterpret_cast<float4 *>(Vb0s);
@@ -436,7 +439,7 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
         lm[slot * 64 + lane] = lrow;
         lm[(KS * QW + slot) * 64 + lane] = m_use;
         __syncthreads();
-        float w[KS], m = -INFINITY, l = 0.0f;
+        float w[KS], m = -3e38f, l = 0.0f;
 #pragma unroll
         for (int h = 0; h < KS; h++) {
             w[h] = lm[(KS * QW + h * QW + wave) * 64 + lane];
