@@ -469,11 +469,12 @@ int aria_hip_qlinear_ex_dev(void *dy, int y_f16, const void *dx, int x_f16, int 
     REQ(M == 0 || N == 0 || (dy && dx && dq && (wtype == ARIA_WF16 || dscale)));
     if (M == 0 || N == 0) return 0;
     hipStream_t s = pick(stream);
-    /* fp32 activations: one conversion pass to fp16 (stream-ordered pool memory), then the
-     * fp16-operand kernel, which stages half the bytes per slice; the value rounded is the
-     * same RTNE half the in-kernel staging would produce */
+    /* fp32 activations that the picked kernel does not take as they are: one conversion pass to fp16
+     * (stream-ordered pool memory), then the fp16-operand kernel, which stages half the bytes per
+     * slice; the value rounded is the same RTNE half the in-kernel rounding produces */
     void *x16 = NULL;
-    if (!x_f16 && K % 32 == 0 && ((uintptr_t)dx & 15u) == 0 &&
+    const int direct = !x_f16 && tiles == 0 && aria_k_qgemm_f32_direct(dy, y_f16, dx, wtype, dq, dscale, db, M, K, N);
+    if (!x_f16 && !direct && K % 32 == 0 && ((uintptr_t)dx & 15u) == 0 &&
         hipMallocAsync(&x16, (size_t)M * K * 2, s) == hipSuccess) {
         hipError_t e = aria_k_f32_to_f16((uint16_t *)x16, (const float *)dx, (size_t)M * K, s);
         if (e == hipSuccess) e = aria_k_qgemm_t(dy, y_f16, x16, 1, wtype, dq, dscale, db, M, K, N, tiles, 0, s);

@@ -836,41 +836,37 @@ void aria_cuda_dit_set_step(aria_cuda_dit *h, int step) {
 /* one velocity evaluation on the handle's buffers (src/aria_sa3_dit.c:734-777):
  * [C,T] -> [T,C]; xtc += preprocess(xtc); seq = [memory tokens | project_in(xtc)];
  * depth blocks; out = project_out(seq[n_mem:]); out += postprocess(out); -> [C,T] */
-/* y [M, N] (+)= x [M, K] . W^T with fp32 x rounded to fp16 in the GEMM's staging and fp16 W,
- * fp32 accumulation and output: the reference's device step runs its four io projections so
- * (gemm_f16w, src/aria_cuda.cu:906-917). add: y += the product (the residual of the pre/post
- * convolutions, x == y), in the epilogue when the MFMA kernel takes the shape and one 128-wide
- * tile covers N (fp32 activations run 128 x 128 tiles), so each workgroup owns whole rows and has
- * read them before it writes them; otherwise through dtmp and k_add. */
-static int io_gemm(aria_cuda_dit *h, float *y, const float *x, const uint16_t *W, int M, int K, int N, int add,
-                   hipStream_t s) {
-    const int mfma = K % 32 == 0 && N % 4 == 0;
-    if (add && mfma && N <= 128) {
-        aria_qgemm_epi e;
-        memset(&e, 0, sizeof e);
-        e.mode = ARIA_EPI_ADD;
-        e.rows_per_batch = M;
-        STEP(aria_k_qgemm_e(y, 0, x, 0, ARIA_WF16, W, NULL, NULL, M, K, N, 0, 0, &e, s), "k_qgemm (io projection)");
-        return 0;
-    }
-    float *dst = add ? h->dtmp : y;
-    STEP(aria_k_qgemm_e(dst, 0, x, 0, ARIA_WF16, W, NULL, NULL, M, K, N, 0, 0, NULL, s), "k_qgemm (io projection)");
-    if (add) STEP(aria_k_add(y, y, dst, (size_t)M * N, s), "k_add (io projection)");
+/* y [M, N] (+)= x [M, K] . W^T with fp32 x rounded to fp16 in the GEMM and fp16 W, fp32
+ * accumulation and output: the reference's device step runs its four io projections so
+ * (gemm_f16w, src/aria_cuda.cu:906-917). add: y += the product, in the epilogue (y and x do not
+ * overlap; K % 32 == 0 and N % 4 == 0, or the fused epilogue is refused). */
+static int io_gemm(float *y, const float *x, const uint16_t *W, int M, int K, int N, int add, hipStream_t s) {
+    aria_qgemm_epi e;
+    memset(&e, 0, sizeof e);
+    e.mode = ARIA_EPI_ADD;
+    e.rows_per_batch = M;
+    STEP(aria_k_qgemm_e(y, 0, x, 0, ARIA_WF16, W, NULL, NULL, M, K, N, 0, 0, add ? &e : NULL, s),
+         "k_qgemm (io projection)");
     return 0;
 }
 
+/* The pre and post convolutions are residual: xtc += pre(xtc), out += post(out). Their GEMMs read
+ * rows that other workgroups would overwrite, so input and result are two buffers: the transpose
+ * before stores the latent twice and the pre-GEMM adds to the copy; the post-GEMM's product is
+ * added by the transpose after it. (Two k_add launches of 5 us each before.) */
 static int step_compute(aria_cuda_dit *h, hipStream_t s) {
     const int B = h->B, T = h->T, S = h->S, C = h->io_ch, E = h->ed, Mt = h->n_mem;
+    const int fuse = h->pre && C % 32 == 0;   /* the MFMA kernels' epilogue adds */
+    float *xin = fuse ? h->dtmp : h->dxtc;
     int rc;
-    STEP(aria_k_transpose(h->dxtc, h->dx, C, T, B, s), "k_transpose (x)");
-    if (h->pre && (rc = io_gemm(h, h->dxtc, h->dxtc, h->pre, B * T, C, C, 1, s))) return rc;
-    for (int b = 0; b < B && Mt; b++)
-        STEP(hipMemcpyAsync(h->dseq + (size_t)b * S * E, h->mem, (size_t)Mt * E * 4, hipMemcpyDeviceToDevice, s),
-             "memory tokens");
+    STEP(aria_k_transpose2(h->dxtc, fuse ? h->dtmp : NULL, h->dx, NULL, C, T, B, s), "k_transpose (x)");
+    if (h->pre && (rc = io_gemm(h->dtmp, h->dxtc, h->pre, B * T, C, C, fuse, s))) return rc;
+    if (h->pre && !fuse) STEP(aria_k_add(h->dxtc, h->dxtc, h->dtmp, (size_t)B * T * C, s), "k_add (io projection)");
+    if (Mt) STEP(aria_k_bcast_rows(h->dseq, (size_t)S * E, h->mem, (size_t)Mt * E, B, s), "memory tokens");
     /* project_in / project_out: one GEMM over both sequences when no memory tokens interleave */
     const int nb = Mt ? B : 1, rows = Mt ? T : B * T;
     for (int b = 0; b < nb; b++)
-        if ((rc = io_gemm(h, h->dseq + ((size_t)b * S + Mt) * E, h->dxtc + (size_t)b * T * C, h->pin, rows, C, E, 0, s)))
+        if ((rc = io_gemm(h->dseq + ((size_t)b * S + Mt) * E, xin + (size_t)b * T * C, h->pin, rows, C, E, 0, s)))
             return rc;
     for (int b = 0; b < h->depth; b++) {
         rc = block_forward(h->blk[b], h->dseq, B, S, h->dgcond, h->ck[b], h->cv[b], h->Sc, h->cos_t, h->sin_t,
@@ -879,10 +875,10 @@ static int step_compute(aria_cuda_dit *h, hipStream_t s) {
         if (rc) return rc;
     }
     for (int b = 0; b < nb; b++)
-        if ((rc = io_gemm(h, h->dout + (size_t)b * T * C, h->dseq + ((size_t)b * S + Mt) * E, h->pout, rows, E, C, 0, s)))
+        if ((rc = io_gemm(h->dout + (size_t)b * T * C, h->dseq + ((size_t)b * S + Mt) * E, h->pout, rows, E, C, 0, s)))
             return rc;
-    if (h->post && (rc = io_gemm(h, h->dout, h->dout, h->post, B * T, C, C, 1, s))) return rc;
-    STEP(aria_k_transpose(h->dv, h->dout, T, C, B, s), "k_transpose (v)");
+    if (h->post && (rc = io_gemm(h->dtmp, h->dout, h->post, B * T, C, C, 0, s))) return rc;
+    STEP(aria_k_transpose2(h->dv, NULL, h->dout, h->post ? h->dtmp : NULL, T, C, B, s), "k_transpose (v)");
     return 0;
 }
 

@@ -78,6 +78,11 @@ hipError_t aria_k_pingpong(float *x, const float *v, const float *noise, float t
 hipError_t aria_k_f32_to_f16(uint16_t *y, const float *x, size_t n, hipStream_t s);
 /* per batch b: dst[b] [cols, rows] = transpose of src[b] [rows, cols] */
 hipError_t aria_k_transpose(float *dst, const float *src, int rows, int cols, int batch, hipStream_t s);
+/* the same of src + add (add NULL: src alone), stored to dst and, unless it is NULL, dst2 */
+hipError_t aria_k_transpose2(float *dst, float *dst2, const float *src, const float *add, int rows, int cols, int batch,
+                             hipStream_t s);
+/* dst + b * dst_stride [n] = src [n] for b < batch (n a multiple of 4, 16-byte aligned) */
+hipError_t aria_k_bcast_rows(float *dst, size_t dst_stride, const float *src, size_t n, int batch, hipStream_t s);
 /* mod[c][b][i] = tssg[c*dim+i] + gcond[b*6*dim + c*dim + i] (gcond may be NULL), c < 6 */
 hipError_t aria_k_mod_chunks(float *mod, const float *tssg, const float *gcond, int B, int dim,
                              hipStream_t s);
@@ -146,6 +151,10 @@ hipError_t aria_k_qgemm(void *y, int y_f16, const void *x, int x_f16, int wtype,
 hipError_t aria_k_qgemm_t(void *y, int y_f16, const void *x, int x_f16, int wtype, const void *q,
                           const float *scale, const float *bias, int M, int K, int N, int tiles,
                           int gelu, hipStream_t s);
+/* 1 when fp32 activations of these arguments go into the GEMM as they are (tiles 0), faster than a
+ * pass that stages them as fp16 first; both give the same rounded operands */
+int aria_k_qgemm_f32_direct(const void *y, int y_f16, const void *x, int wtype, const void *q,
+                            const float *scale, const float *bias, int M, int K, int N);
 /* the same with a fused epilogue (epi NULL = STORE); HEADS needs N % 64 == 0 */
 hipError_t aria_k_qgemm_e(void *y, int y_f16, const void *x, int x_f16, int wtype, const void *q,
                           const float *scale, const float *bias, int M, int K, int N, int tiles,

@@ -293,25 +293,48 @@ extern "C" hipError_t aria_k_pingpong(float *x, const float *v, const float *noi
 
 /* batched 2-D transpose through a 32x33 LDS tile: dst[b][c][r] = src[b][r][c]
  * (the DiT step's [C,T] <-> [T,C] latent reshapes, src/aria_sa3_dit.c:585-597) */
-__global__ __launch_bounds__(256) void k_transpose(float *dst, const float *src, int rows, int cols) {
+__global__ __launch_bounds__(256) void k_transpose(float *dst, float *dst2, const float *src, const float *add,
+                                                    int rows, int cols) {
     __shared__ float t[32][33];
     const size_t base = (size_t)blockIdx.z * rows * cols;
     const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   /* 32 x 8 threads */
     for (int i = ty; i < 32; i += 8) {
         const int r = r0 + i, c = c0 + tx;
-        if (r < rows && c < cols) t[i][tx] = src[base + (size_t)r * cols + c];
+        const size_t at = base + (size_t)r * cols + c;
+        if (r < rows && c < cols) t[i][tx] = add ? src[at] + add[at] : src[at];
     }
     __syncthreads();
     for (int i = ty; i < 32; i += 8) {
         const int c = c0 + i, r = r0 + tx;
-        if (r < rows && c < cols) dst[base + (size_t)c * rows + r] = t[tx][i];
+        if (r < rows && c < cols) {
+            const size_t at = base + (size_t)c * rows + r;
+            dst[at] = t[tx][i];
+            if (dst2) dst2[at] = t[tx][i];
+        }
     }
 }
-extern "C" hipError_t aria_k_transpose(float *dst, const float *src, int rows, int cols, int batch, hipStream_t s) {
+extern "C" hipError_t aria_k_transpose2(float *dst, float *dst2, const float *src, const float *add, int rows, int cols,
+                                        int batch, hipStream_t s) {
     if (rows <= 0 || cols <= 0 || batch <= 0) return hipSuccess;
     dim3 grid((cols + 31) / 32, (rows + 31) / 32, batch);
-    hipLaunchKernelGGL(k_transpose, grid, dim3(256), 0, s, dst, src, rows, cols);
+    hipLaunchKernelGGL(k_transpose, grid, dim3(256), 0, s, dst, dst2, src, add, rows, cols);
+    return hipGetLastError();
+}
+extern "C" hipError_t aria_k_transpose(float *dst, const float *src, int rows, int cols, int batch, hipStream_t s) {
+    return aria_k_transpose2(dst, nullptr, src, nullptr, rows, cols, batch, s);
+}
+
+/* one source row set to every sequence of a batch (the DiT's memory tokens in front of each): one
+ * launch of ~2 us where a device copy per sequence took ~5 us each */
+__global__ __launch_bounds__(256) void k_bcast_rows(float4 *dst, size_t stride4, const float4 *src, size_t n4) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) dst[blockIdx.y * stride4 + i] = src[i];
+}
+extern "C" hipError_t aria_k_bcast_rows(float *dst, size_t dst_stride, const float *src, size_t n, int batch, hipStream_t s) {
+    if (n == 0 || batch <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_bcast_rows, dim3((unsigned)((n / 4 + 255) / 256), batch), dim3(256), 0, s, (float4 *)dst,
+                       dst_stride / 4, (const float4 *)src, n / 4);
     return hipGetLastError();
 }
 

@@ -9,7 +9,9 @@
  * life of the process. Its device address is resolved once per device with
  * hipGetSymbolAddress (host code sees only a stand-in for the array's name), at library init
  * for the library's device and on the first call on any other, and kept per device; every
- * kernel argument and copy uses that address.
+ * kernel argument and copy uses that address. Calls whose GEMM takes the fp32 activations as they
+ * are (aria_k_qgemm_f32_direct: few output tiles) stage nothing and need no ordering; a staging
+ * size above the scratch is refused whichever kernel the shape has.
  *
  * Every call on one GPU shares that GPU's array and the array keeps the last call's
  * contents. The staging is fully written before the GEMM reads it, so nothing needs
@@ -100,6 +102,9 @@ extern "C" int aria_hip_qlinear_noalloc_dev(void *dy, int y_f16, const void *dx,
                                M, K, need, (size_t)ARIA_HIP_NOALLOC_SCRATCH);
             return ARIA_HIP_EINVAL;
         }
+    }
+    if (!x_f16 && K % 32 == 0 && ((uintptr_t)dx & 15u) == 0 &&
+        !aria_k_qgemm_f32_direct(dy, y_f16, dx, wtype, dq, dscale, db, M, K, N)) {
         std::lock_guard<std::mutex> lk(g_mu);
         void *p = nullptr;
         int dev = 0;

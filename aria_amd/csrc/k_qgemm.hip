@@ -447,14 +447,42 @@ int qgemm_pick(int wt, bool heads, int M, int N, int K, int cur) {
     return best;
 }
 
+static bool qgemm_aligned(const QArgs &a, int wt) {
+    return a.K % BK == 0 && a.N % 4 == 0 && ((uintptr_t)a.x & 15u) == 0 && ((uintptr_t)a.q & 15u) == 0 &&
+           ((uintptr_t)a.y & 15u) == 0 && (a.bias == nullptr || ((uintptr_t)a.bias & 15u) == 0) &&
+           (wt != ARIA_WQ8 || ((uintptr_t)a.scale & 15u) == 0) && (wt != ARIA_WQ4 || ((uintptr_t)a.scale & 7u) == 0);
+}
+
+/* fp32 activations straight into the K-split kernel: its configuration (the first of 32 x 32, 32 x 64
+ * and 64 x 64 whose tiles fit one round of the 256 CUs), or -1. It reads twice the activation bytes
+ * per tile, and saves the staging pass (a launch of 3 us and one more dependent kernel) or, where
+ * there is none, the 128 x 128 tiles of the LDS-operand kernel (few workgroups, each a serial chain
+ * of K / 32 slices). Measured in us, fp16 weights, (M, K, N), staged / LDS-operand / direct:
+ * (172, 1024, 1024) 6.9 / 16.7 / 4.9; (1024, 1024, 1024) 11.5 / 17.4 / 10.2; (256, 1024, 3072)
+ * 10.2 / 17.3 / 9.0; (108, 256, 1024) 5.3 / 7.4 / 3.2; (1292, 1024, 256) 9.4 / 17.1 / 7.4. Past one
+ * round it loses ((344, 1024, 3072) 12.6 / 17.3 / 14.8), and so it does on long chains: at K = 4096
+ * (172, 4096, 1024) 11.4 / 49.0 / 11.9, so the line is drawn at twice the K that gains 2 us.
+ * An output that overlaps the activations keeps the staging pass: its copy is what lets one
+ * workgroup store rows that another has yet to read. */
+static int qgemm_f32_pick(const QArgs &a, int wt) {
+    if (a.K % 64 || a.K > 2048 || !qgemm_aligned(a, wt) || (wt == ARIA_WQ4 && ((uintptr_t)a.scale & 15u))) return -1;
+    const uintptr_t x0 = (uintptr_t)a.x, y0 = (uintptr_t)a.y;
+    if (x0 < y0 + (size_t)a.M * a.N * (a.y_f16 ? 2 : 4) && y0 < x0 + (size_t)a.M * a.K * 4) return -1;
+    const long long m32 = (a.M + 31) / 32, m64 = (a.M + 63) / 64, n32 = (a.N + 31) / 32, n64 = (a.N + 63) / 64;
+    return m32 * n32 <= 256 ? 0 : m32 * n64 <= 256 ? 1 : m64 * n64 <= 256 ? 2 : -1;
+}
+
+extern "C" int aria_k_qgemm_f32_direct(const void *y, int y_f16, const void *x, int wtype, const void *q, const float *scale,
+                                       const float *bias, int M, int K, int N) {
+    QArgs a;
+    memset(&a, 0, sizeof a);
+    a.y = (void *)y; a.y_f16 = y_f16; a.x = x; a.q = q; a.scale = scale; a.bias = bias; a.M = M; a.K = K; a.N = N;
+    return qgemm_f32_pick(a, wtype) >= 0;
+}
+
 template <int WT, bool AF16>
 static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
-    const bool aligned = a.K % BK == 0 && a.N % 4 == 0 && ((uintptr_t)a.x & 15u) == 0 &&
-                         ((uintptr_t)a.q & 15u) == 0 && ((uintptr_t)a.y & 15u) == 0 &&
-                         (a.bias == nullptr || ((uintptr_t)a.bias & 15u) == 0) &&
-                         (WT != ARIA_WQ8 || ((uintptr_t)a.scale & 15u) == 0) &&
-                         (WT != ARIA_WQ4 || ((uintptr_t)a.scale & 7u) == 0);
-    if (!aligned) {
+    if (!qgemm_aligned(a, WT)) {
         if (a.epi.mode != ARIA_EPI_STORE) return hipErrorInvalidValue;   /* fused epilogues need the MFMA path */
         dim3 grid((a.N + 63) / 64, (a.M + 63) / 64);
         hipLaunchKernelGGL((k_qgemm_simt<WT, AF16>), grid, dim3(256), 0, s, a);
@@ -462,6 +490,10 @@ static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
     }
     if constexpr (!AF16) {   /* fp32 activations: the fallback when no fp16 staging buffer was available */
         if (a.epi.mode == ARIA_EPI_HEADS) return hipErrorInvalidValue;
+        if (tiles >= GEMM_KS) return qgemm_ks_f32_launch(a, WT, tiles - GEMM_KS, s);
+        const bool plain = !a.gelu && (a.epi.mode == ARIA_EPI_STORE || a.epi.mode == ARIA_EPI_ADD);
+        const int c = tiles == 0 && plain ? qgemm_f32_pick(a, WT) : -1;
+        if (c >= 0) return qgemm_ks_f32_launch(a, WT, c, s);
         launch_cfg<C2, WT, AF16>(a, s);
         return hipGetLastError();
     } else {

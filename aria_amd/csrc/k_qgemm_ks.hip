@@ -37,22 +37,23 @@ __device__ __forceinline__ int swz(int r) {
 
 /* one K-tile of one wave in LDS (bytes): RB bytes of each activation row, and the weight rows'
  * share of the same k */
-template <int WT, int FM, int FN, int RB>
+template <int WT, int FM, int FN, int RB, bool AF32>
 struct KStage {
+    static_assert(!AF32 || (WT != ARIA_WI8 && RB == 128), "fp32 activations: 32 k per K-tile");
     static constexpr bool WIDE = WT == ARIA_WI8 || WT == ARIA_WF16;
-    static constexpr int WB = WIDE ? RB : WT == ARIA_WQ8 ? RB / 2 : RB / 4;   /* bytes of a weight row */
+    static constexpr int KK = WT == ARIA_WI8 ? RB : AF32 ? RB / 4 : RB / 2;   /* k per K-tile */
+    static constexpr int NK = KK / (WT == ARIA_WI8 ? 32 : 16);                /* MFMA steps per K-tile */
+    static constexpr int WB = WT == ARIA_WF16 ? 2 * KK : WT == ARIA_WQ4 ? KK / 2 : KK;   /* bytes of a weight row */
     static constexpr int A = 32 * FM * RB;
     static constexpr int NQ = (32 * FN * WB + 1023) / 1024, NS = WT == ARIA_WQ4 ? (FN + 1) / 2 : 0;
     static constexpr int WQ = NQ * 1024, WS = NS * 1024;   /* WS: [min, step] pairs, 16 B per row */
     static constexpr int BYTES = A + WQ + WS;
     static constexpr int NA = A / 1024, DMA = NA + NQ + NS;   /* transfers of 1 KB */
-    static constexpr int KK = WT == ARIA_WI8 ? RB : RB / 2;   /* k per K-tile */
-    static constexpr int NK = RB / 32;                        /* MFMA steps per K-tile */
 };
 
-template <int WT, int FM, int FN, int KW, int RB>
+template <int WT, int FM, int FN, int KW, int RB, bool AF32>
 struct KCfg {
-    using St = KStage<WT, FM, FN, RB>;
+    using St = KStage<WT, FM, FN, RB, AF32>;
     static constexpr int ESTR = 32 * FN * 4 + 16;       /* partial-sum row stride (padded by 16 B) */
     static constexpr int PART = 32 * ESTR;              /* one wave's partial sums of a 32-row group */
     /* stages: as many (up to four) as the LDS share of PW workgroups per CU allows */
@@ -235,11 +236,11 @@ __device__ __forceinline__ void row_epilogue(const QArgs &a, float (&v)[NU][4], 
 
 }  // namespace
 
-template <int WT, int FM, int FN, int KW, int RB>
-__global__ __launch_bounds__(64 * KW) __attribute__((amdgpu_waves_per_eu(KW * KCfg<WT, FM, FN, KW, RB>::PW / 4))) void
+template <int WT, int FM, int FN, int KW, int RB, bool AF32>
+__global__ __launch_bounds__(64 * KW) __attribute__((amdgpu_waves_per_eu(KW * KCfg<WT, FM, FN, KW, RB, AF32>::PW / 4))) void
 k_qgemm_ks(QArgs a, int MT, int T) {
-    using C = KCfg<WT, FM, FN, KW, RB>;
-    using St = KStage<WT, FM, FN, RB>;
+    using C = KCfg<WT, FM, FN, KW, RB, AF32>;
+    using St = KStage<WT, FM, FN, RB, AF32>;
     constexpr int NST = C::NST, NK = St::NK, WB = St::WB;
     __shared__ __attribute__((aligned(16))) uint8_t smem[KW * C::REG];
 
@@ -258,7 +259,7 @@ k_qgemm_ks(QArgs a, int MT, int T) {
     /* per-lane sources of the transfers for K-tile 0. Rows past the edge re-read the last one:
      * their products land in rows or columns that are never stored */
     const uint8_t *xsrc[St::NA], *wsrc[St::NQ], *ssrc[St::NS ? St::NS : 1];
-    constexpr int XB = WT == ARIA_WI8 ? 1 : 2;   /* bytes per activation */
+    constexpr int XB = WT == ARIA_WI8 ? 1 : AF32 ? 4 : 2;   /* bytes per activation */
     /* transfer i fills rows (1024 / row bytes) i ..: lane -> row and stored chunk */
 #pragma unroll
     for (int i = 0; i < St::NA; i++) {
@@ -281,10 +282,10 @@ k_qgemm_ks(QArgs a, int MT, int T) {
         for (int i = 0; i < St::NA; i++) dma16(xsrc[i] + (size_t)kt * RB, b + 1024 * i);
 #pragma unroll
         for (int i = 0; i < St::NQ; i++) dma16(wsrc[i] + (size_t)kt * WB, b + St::A + 1024 * i);
-        if constexpr (WT == ARIA_WQ4) {   /* the pairs of 64 k: this K-tile's, with RB = 64 also its neighbour's */
+        if constexpr (WT == ARIA_WQ4) {   /* the pairs of 64 k: this K-tile's, with 32 k also its neighbour's */
 #pragma unroll
             for (int i = 0; i < St::NS; i++)
-                dma16(ssrc[i] + (size_t)(RB == 64 ? kt >> 1 : kt) * 16, b + St::A + St::WQ + 1024 * i);
+                dma16(ssrc[i] + (size_t)(St::KK == 32 ? kt >> 1 : kt) * 16, b + St::A + St::WQ + 1024 * i);
         }
     };
 
@@ -303,10 +304,14 @@ k_qgemm_ks(QArgs a, int MT, int T) {
     for (int p = 0; p < NST; p++)
         if (p < nt) issue(p, wave + p * KW);
 
-    /* fragment offsets: step s of lane half lh reads chunk NK lh + s of row lrow */
-    int aoff[NK];
+    /* fragment offsets: step s of lane half lh reads chunk NK lh + s of row lrow (fp32 activations:
+     * the 32 bytes of its eight k, two chunks) */
+    int aoff[NK * (AF32 ? 2 : 1)], woff[NK];
 #pragma unroll
-    for (int k = 0; k < NK; k++) aoff[k] = lrow * RB + 16 * ((NK * lh + k) ^ swz<RB>(lrow));
+    for (int k = 0; k < NK * (AF32 ? 2 : 1); k++)
+        aoff[k] = lrow * RB + 16 * (((AF32 ? 2 : 1) * NK * lh + k) ^ swz<RB>(lrow));
+#pragma unroll
+    for (int k = 0; k < NK; k++) woff[k] = lrow * WB + 16 * ((NK * lh + k) ^ swz<WB>(lrow));
     int st = 0;
     for (int i = 0; i < nt; i++) {
         /* this tile's transfers are the oldest in flight; up to NST - 1 tiles follow them */
@@ -323,13 +328,21 @@ k_qgemm_ks(QArgs a, int MT, int T) {
 #pragma unroll
         for (int k = 0; k < NK; k++)
 #pragma unroll
-            for (int m = 0; m < FM; m++) xf[k][m] = *reinterpret_cast<const FragT *>(S + 32 * RB * m + aoff[k]);
+            for (int m = 0; m < FM; m++) {
+                if constexpr (AF32) {   /* rounded to fp16 as the staging pass rounds them */
+                    const float4 u = *reinterpret_cast<const float4 *>(S + 32 * RB * m + aoff[2 * k]);
+                    const float4 v = *reinterpret_cast<const float4 *>(S + 32 * RB * m + aoff[2 * k + 1]);
+                    xf[k][m] = __builtin_bit_cast(FragT, make_uint4(pack2h(u.x, u.y), pack2h(u.z, u.w), pack2h(v.x, v.y), pack2h(v.z, v.w)));
+                } else {
+                    xf[k][m] = *reinterpret_cast<const FragT *>(S + 32 * RB * m + aoff[k]);
+                }
+            }
 #pragma unroll
         for (int j = 0; j < FN; j++) {
             const int r = 32 * j + lrow;
             if constexpr (St::WIDE) {
 #pragma unroll
-                for (int k = 0; k < NK; k++) wf[k][j] = *reinterpret_cast<const FragT *>(S + St::A + 32 * RB * j + aoff[k]);
+                for (int k = 0; k < NK; k++) wf[k][j] = *reinterpret_cast<const FragT *>(S + St::A + 32 * WB * j + woff[k]);
             } else if constexpr (WT == ARIA_WQ8) {
 #pragma unroll
                 for (int k = 0; k < NK / 2; k++) {
@@ -344,7 +357,7 @@ k_qgemm_ks(QArgs a, int MT, int T) {
                     const uint2 u = *reinterpret_cast<const uint2 *>(S + St::A + r * WB + 8 * lh);
                     qw[j][0] = u.x; qw[j][1] = u.y;
                 }
-                pr[j] = *reinterpret_cast<const uint2 *>(S + St::A + St::WQ + 16 * r + 8 * (RB == 64 ? kt & 1 : lh));
+                pr[j] = *reinterpret_cast<const uint2 *>(S + St::A + St::WQ + 16 * r + 8 * (St::KK == 32 ? kt & 1 : lh));
             }
         }
         /* every read of this stage has returned before its next transfers are issued */
@@ -463,10 +476,10 @@ k_qgemm_ks(QArgs a, int MT, int T) {
     }
 }
 
-template <int WT, int FM, int FN, int KW, int RB>
+template <int WT, int FM, int FN, int KW, int RB, bool AF32 = false>
 static void launch_ks(const QArgs &a, hipStream_t s) {
     const int MT = (a.M + 32 * FM - 1) / (32 * FM), T = MT * ((a.N + 32 * FN - 1) / (32 * FN));
-    hipLaunchKernelGGL((k_qgemm_ks<WT, FM, FN, KW, RB>), dim3((T + 7) / 8 * 8), dim3(64 * KW), 0, s, a, MT, T);
+    hipLaunchKernelGGL((k_qgemm_ks<WT, FM, FN, KW, RB, AF32>), dim3((T + 7) / 8 * 8), dim3(64 * KW), 0, s, a, MT, T);
 }
 
 /* the configurations compiled: 32-row blocks, 32-column blocks, waves, bytes of an activation row
@@ -484,6 +497,25 @@ static void launch_ks(const QArgs &a, hipStream_t s) {
 #define KS_CFGS(X) X(0, 1, 1, 8, 128) X(1, 1, 2, 8, 128) X(2, 2, 2, 4, 128) X(3, 3, 2, 4, 128) X(4, 2, 2, 4, 64)
 static const int ks_fn[] = {1, 2, 2, 2, 2};
 int qgemm_ks_ncfg() { return (int)(sizeof ks_fn / sizeof ks_fn[0]); }
+
+template <int WT>
+static hipError_t launch_ks_f32(const QArgs &a, int cfg, hipStream_t s) {
+    if (cfg == 0) launch_ks<WT, 1, 1, 8, 128, true>(a, s);
+    else if (cfg == 1) launch_ks<WT, 1, 2, 8, 128, true>(a, s);
+    else if (cfg == 2) launch_ks<WT, 2, 2, 4, 128, true>(a, s);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t qgemm_ks_f32_launch(const QArgs &a, int wt, int cfg, hipStream_t s) {
+    if (a.K % 64 || (a.gelu && a.epi.mode != ARIA_EPI_STORE) || (a.epi.mode != ARIA_EPI_STORE && a.epi.mode != ARIA_EPI_ADD) ||
+        (wt == ARIA_WQ4 && ((uintptr_t)a.scale & 15u)))
+        return hipErrorInvalidValue;
+    if (wt == ARIA_WQ8) return launch_ks_f32<ARIA_WQ8>(a, cfg, s);
+    if (wt == ARIA_WQ4) return launch_ks_f32<ARIA_WQ4>(a, cfg, s);
+    if (wt == ARIA_WF16) return launch_ks_f32<ARIA_WF16>(a, cfg, s);
+    return hipErrorInvalidValue;
+}
 
 hipError_t qgemm_ks_launch(const QArgs &a, int wt, int cfg, hipStream_t s) {
     if (a.K % (wt == ARIA_WI8 ? 128 : 64) || cfg < 0 || cfg >= qgemm_ks_ncfg() || (a.gelu && a.epi.mode != ARIA_EPI_STORE) ||

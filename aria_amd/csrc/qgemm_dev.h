@@ -475,6 +475,9 @@ int qgemm_big_i8_ncfg();
  * ARIA_WQ8, ARIA_WQ4, ARIA_WF16 (fp16 activations) or ARIA_WI8 (int8 ones), K % 64 == 0 */
 hipError_t qgemm_ks_launch(const QArgs &a, int wt, int cfg, hipStream_t s);
 int qgemm_ks_ncfg();
+/* the same with fp32 activations, rounded to fp16 as fragments are read (configurations 0 .. 2,
+ * STORE and ADD) */
+hipError_t qgemm_ks_f32_launch(const QArgs &a, int wt, int cfg, hipStream_t s);
 /* the kernel for an M x N product of depth K: `cur` (a k_qgemm_big.hip configuration of this
  * weight type, the pick at M = 2592) or another one of them, or GEMM_KS + a k_qgemm_ks.hip
  * configuration (k_qgemm.hip) */
