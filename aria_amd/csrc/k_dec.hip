@@ -8,9 +8,9 @@
  *   k_dec_in      softnorm inverse and transpose: latent [256, T] * std -> fp16 [T, 256]
  *   k_dec_expand  the 17-token groups: frame t's projected token, then 16 new_tokens
  *   k_dec_dyt     DynamicTanh norm tanh(alpha x) * gamma + beta -> fp16 GEMM operand
- *   k_dec_attn_mfma  one chunk-head of the differential self-attention, fused: both
- *                 softmax(q k^T / 8) v products over the chunk's 34 tokens on the fp32 MFMA,
- *                 their difference, merged fp16 (the q/k DynamicTanh norms and RoPE, 32
+ *   k_dec_attn_mfma  one chunk-head of the differential self-attention, fused: the
+ *                 difference of two softmax(q k^T / 8) over the chunk's 34 tokens, times v,
+ *                 on the fp32 MFMA, merged fp16 (the q/k DynamicTanh norms and RoPE, 32
  *                 rotated dims, are the to_qkv GEMM's DYT_ROPE epilogue)
  *   k_dec_split   the k = 3 mapping convolution's input rows (the last 16 of each group), every
  *                 value split into three bf16 parts
@@ -80,170 +80,147 @@ struct DecAttnArgs {
 };
 
 /* ---- the chunk attention on the fp32 MFMA (v_mfma_f32_16x16x4_f32) ----
- * One (chunk, head) per workgroup of six waves; wave w computes pair p = w / 3 (0: q, k;
- * 1: qd, kd) for the 16 queries of block i = w % 3 of the chunk's 34 tokens padded to 48
- * (3 blocks of 16). The q / k sections of qkv arrive DynamicTanh-normed and rotated (the
- * to_qkv GEMM's DYT_ROPE epilogue, once per element). Against one wave per pair (288 MFMAs in
- * one wave's chain, 129 VGPRs, three waves per SIMD) each wave runs 96 MFMAs at 58 VGPRs:
- * decode 0.698 -> 0.686 ms at T = 108, 2.71 -> 2.63 ms at T = 646, same bits.
- *   v (34 rows x 64 dims, shared by all six waves) travels to LDS by LDS DMA first thing, so
- *     its fetch overlaps the q / k loads and takes no registers
- *   each wave loads its block's 16 q rows and 16 k rows once; the k rows go through LDS to the
- *     pair's other two waves (loading all 48 per wave doubled the L2 reads: slower at T = 2584)
- *   S = q k^T for the wave's query block: 1 x 3 blocks, 16 k-steps; lane l supplies row l % 16
- *     of q (A) and of k (B) at dim 16 (l / 16) + s in step s (16 consecutive dims of one row)
- *   softmax over the 34 valid keys in the accumulators (a row's 16 columns of a block sit in
- *     16 lanes: xor-shuffle reductions), probabilities through the wave's own 16 LDS rows
- *     (over the k space, once every wave's k reads are done) into the A layout
- *   O = P v: 1 x 4 blocks, 12 k-steps over keys 12 (l / 16) + s; output block j column n
- *     holds dim 4 n + j, so a lane's B operands of a step are one 16-byte LDS read of v and
- *     its four output dims of a row are adjacent (one 8-byte store)
- * The pair-1 waves leave O in LDS (lane-major, over the v space once every product is done),
- * the pair-0 wave of the same block writes half(O0 - O1) to the merged rows. Accumulator v of
- * lane l in a 16 x 16 block: row 4 (l / 16) + v, column l % 16. Padded q / k rows are zero and
- * padded keys are masked before the max and multiply zero v, so nothing past the chunk's rows
- * is used. Every output element is the same sequence of operations as with one wave per pair.
+ * One (chunk, head) per workgroup of three waves; wave w computes the 16 queries of block w of
+ * the chunk's 34 tokens (padded to 48) for both pairs (q, k and qd, kd). The q / k sections of
+ * qkv arrive DynamicTanh-normed and rotated (the to_qkv GEMM's DYT_ROPE epilogue).
+ *   k, kd and v (34 rows of 256 B each) travel to LDS by LDS DMA first thing, in whole rows; the
+ *     16-byte chunk c of LDS row R sits at slot c ^ (R % 16), so 16 lanes that read one chunk of
+ *     16 rows, or one whole row, meet no bank twice
+ *   S^T = k q^T (keys are the rows): lane l supplies key row l % 16 (A) and query l % 16 (B) at
+ *     dims 16 j + 4 (l / 16) + e in step (j, e), so 16-byte reads feed four steps, and query l %
+ *     16's scores of keys 16 b + 4 (l / 16) + v end up in the accumulators of its four lanes: the
+ *     softmax is 9 values a lane and two lane swaps, and a probability is already where the second
+ *     product wants it (k = l / 16, column l % 16), with no pass through LDS
+ *   O = (P0 - P1) v, one product for the two pairs' difference: O^T = v^T D^T, step (b, v) over
+ *     keys 16 b + 4 (l / 16) + v; output block j row m holds dim 4 m + j, so a lane's A operands
+ *     of a step are one 16-byte read of v and its 16 outputs are dims 16 (l / 16) .. of one query
+ *   keys 32 and 33 would fill two of 16 rows of a third block: their scores are summed on the VALU
+ *     (each lane its 16 dims, then over the four lanes), and in the second product they share one
+ *     step (lq 0 and 1)
+ * Memory bounds it at T = 646: 168 MB of fp32 qkv and 17 MB of output are 38 us at the rate of a
+ * large copy. One wave per (pair, query block) with k and P through LDS, two products and scattered
+ * 16-byte loads took 69 us there (576 MFMAs a workgroup, 300 now) and 16.5 us at T = 108; this form
+ * 44 and 12.3 (46.5 and 13.4 with a third key block on the MFMA). Relative error against float64 is
+ * the fp16 output's, 2.07e-4 before and now.
  * fp32 operands, as the reference keeps this attention fp32. */
-#define DA_P 48            /* padded chunk */
-#define DA_PS 52           /* LDS row stride of P (floats; 16-byte aligned rows) */
-#define DA_KS 68           /* LDS row stride of k (floats; rows spread over the banks) */
-#define DA_VCH 576         /* v staging: 16-byte chunks (34 rows x 16, rounded up to 9 x 64) */
-#define DA_WAVES 6
+#define DA_WAVES 3
+#define DA_ROWS (3 * DEC_S)                       /* k, kd, v */
+#define DA_DMA ((DA_ROWS * 16 + 63) / 64)         /* transfers of 64 16-byte chunks */
 
 typedef float f32x4_dec __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) float4 lds_f4_dec;
 
-/* this lane's 16 dims (16 lq ..) of row r of the section at column off; rows past the chunk
- * are zero */
-__device__ __forceinline__ void dec_ld_row(float (&f)[16], const float *base, int off, int r, int lq) {
-    const bool ok = r < DEC_S;
-    const float *row = base + (size_t)(ok ? r : 0) * DEC_QKV + off + lq * 16;
-#pragma unroll
-    for (int j4 = 0; j4 < 4; j4++) {
-        const float4 x = *reinterpret_cast<const float4 *>(row + 4 * j4);
-        f[4 * j4 + 0] = ok ? x.x : 0.0f; f[4 * j4 + 1] = ok ? x.y : 0.0f;
-        f[4 * j4 + 2] = ok ? x.z : 0.0f; f[4 * j4 + 3] = ok ? x.w : 0.0f;
-    }
+/* over the four lanes l % 16 + {0, 16, 32, 48} */
+template <typename Op>
+__device__ __forceinline__ float dec_quad(float v, Op op) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned a = r[0], b = r[1];
+    const float w = op(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    const unsigned u2 = __builtin_bit_cast(unsigned, w);
+    const auto t = __builtin_amdgcn_permlane32_swap(u2, u2, false, false);
+    const unsigned c = t[0], d = t[1];
+    return op(__builtin_bit_cast(float, c), __builtin_bit_cast(float, d));
 }
 
 __global__ __launch_bounds__(64 * DA_WAVES) void k_dec_attn_mfma(DecAttnArgs a, int H) {
-    /* [0, 9216): v rows (256 B each); then k of both pairs (2 x 48 rows x 68 floats), later
-     * reused for P (6 waves x 16 rows x 52); after every product: O of the pair-1 waves (3 x
-     * 16 x 64 floats, lane-major) from offset 0 */
-    __shared__ __attribute__((aligned(16))) float sm[DA_VCH * 4 + 2 * 48 * DA_KS];
-    static_assert(2 * 48 * DA_KS >= DA_WAVES * 16 * DA_PS, "P fits the k space");
-    float4 *Vs = reinterpret_cast<float4 *>(sm);
+    __shared__ __attribute__((aligned(16))) float4 sm[DA_DMA * 64];
     const int ch = blockIdx.x / H, h = blockIdx.x % H;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int pair = wave / 3, qi = wave % 3;
     const int lr = lane & 15, lq = lane >> 4;
     const float *base = a.qkv + (size_t)ch * DEC_S * DEC_QKV + h * DEC_HD;
 
-    /* v by LDS DMA: instruction i moves chunks 64 i .. 64 i + 63 (row p / 16, dims 4 (p % 16)
-     * ..), wave w the instructions i = w, w + 6; chunks past the 34 rows re-read row 33 */
-    {
-        typedef __attribute__((address_space(3))) void lds_void_t;
-        for (int i = wave; i < DA_VCH / 64; i += DA_WAVES) {
-            const int p = 64 * i + lane, r = min(p >> 4, DEC_S - 1);
-            __builtin_amdgcn_global_load_lds(base + (size_t)r * DEC_QKV + 1536 + 4 * (p & 15),
-                                             (lds_void_t *)(sm + 256 * i), 16, 0, 0);
-        }
+    /* transfer i fills slots 64 i ..; slots past the last row re-read it */
+    for (int i = wave; i < DA_DMA; i += DA_WAVES) {
+        const int p = 64 * i + lane, R = min(p >> 4, DA_ROWS - 1);
+        const int sec = R >= 2 * DEC_S ? 2 : R >= DEC_S;
+        const float *src = base + (size_t)(R - sec * DEC_S) * DEC_QKV + (sec == 2 ? 1536 : sec ? 3072 : 768);
+        dma16(src + 4 * ((p ^ R) & 15), (uint32_t)(uintptr_t)(lds_f4_dec *)sm + 1024 * i);
     }
-    /* q (or qd) rows 16 qi + lr in registers; k (or kd) rows 16 qi + lr through LDS to the
-     * pair's three waves */
-    float qf[16], kf[3][16];
-    float *Ks = sm + DA_VCH * 4 + pair * (48 * DA_KS);
-    {
-        float kr[16];
-        dec_ld_row(qf, base, pair ? 2304 : 0, qi * 16 + lr, lq);
-        dec_ld_row(kr, base, pair ? 3072 : 768, qi * 16 + lr, lq);
+    /* the wave's query (rows past the chunk repeat the last one; they are not stored) */
+    const int qrow = 16 * wave + lr;
+    float4 qf[2][4];
 #pragma unroll
-        for (int j4 = 0; j4 < 4; j4++)
-            *reinterpret_cast<float4 *>(Ks + (qi * 16 + lr) * DA_KS + lq * 16 + 4 * j4) =
-                make_float4(kr[4 * j4], kr[4 * j4 + 1], kr[4 * j4 + 2], kr[4 * j4 + 3]);
+    for (int p = 0; p < 2; p++) {
+        const float *row = base + (size_t)min(qrow, DEC_S - 1) * DEC_QKV + (p ? 2304 : 0) + 4 * lq;
+#pragma unroll
+        for (int j = 0; j < 4; j++) qf[p][j] = *reinterpret_cast<const float4 *>(row + 16 * j);
     }
-    __syncthreads();   /* the pair's 48 k rows in LDS */
-#pragma unroll
-    for (int bk = 0; bk < 3; bk++)
-#pragma unroll
-        for (int j4 = 0; j4 < 4; j4++) {
-            const float4 k4 = *reinterpret_cast<const float4 *>(Ks + (bk * 16 + lr) * DA_KS + lq * 16 + 4 * j4);
-            kf[bk][4 * j4] = k4.x; kf[bk][4 * j4 + 1] = k4.y; kf[bk][4 * j4 + 2] = k4.z; kf[bk][4 * j4 + 3] = k4.w;
-        }
-    /* S = q k^T for the wave's query block */
-    f32x4_dec sc[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) sc[j] = f32x4_dec{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int st = 0; st < 16; st++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) sc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[st], kf[j][st], sc[j], 0, 0, 0);
-    __syncthreads();   /* every wave's k reads done before P overwrites them */
+    wait_vm<0>();
+    __syncthreads();   /* k, kd and v in LDS */
 
-    /* softmax of each row over keys < 34 (block 2 holds keys 32 + lr) */
-    float *P = sm + DA_VCH * 4 + wave * (16 * DA_PS);
+    f32x4_dec sc[2][2];
+    float st[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};   /* keys 32 and 33: this lane's dims */
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        float x0 = sc[0][v] * 0.125f, x1 = sc[1][v] * 0.125f;
-        float x2 = lr < DEC_S - 32 ? sc[2][v] * 0.125f : -INFINITY;
-        float mx = fmaxf(fmaxf(x0, x1), x2);
-        mx = grp_max<16>(mx);   /* DPP within the row of 16 lanes, no LDS round trip */
-        x0 = exp_fast(x0 - mx); x1 = exp_fast(x1 - mx); x2 = exp_fast(x2 - mx);
-        float sum = (x0 + x1) + x2;
-        sum = grp_sum<16>(sum);
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) sc[p][b] = f32x4_dec{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float4 kf[2][2], kt[2][2];
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const int R = p * DEC_S + 16 * b + lr, Rt = p * DEC_S + 32 + b;
+                kf[p][b] = sm[R * 16 + (((4 * j + lq) ^ R) & 15)];
+                kt[p][b] = sm[Rt * 16 + (((4 * j + lq) ^ Rt) & 15)];
+            }
+#define DA_STEP(c)                                                                                            \
+        _Pragma("unroll") for (int p = 0; p < 2; p++)                                                         \
+            _Pragma("unroll") for (int b = 0; b < 2; b++)                                                     \
+                st[p][b] = __builtin_fmaf(kt[p][b].c, qf[p][j].c, st[p][b]),                                  \
+                sc[p][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[p][b].c, qf[p][j].c, sc[p][b], 0, 0, 0);
+        DA_STEP(x) DA_STEP(y) DA_STEP(z) DA_STEP(w)
+#undef DA_STEP
+    }
+
+    /* softmax over the 34 keys: eight in the accumulators, the last two as a ninth value of lq 0 and 1 */
+    float D[9];
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        float x[9];
+#pragma unroll
+        for (int i = 0; i < 8; i++) { const float t = sc[p][i >> 2][i & 3]; x[i] = t * 0.125f; }
+        const float t0 = dec_quad(st[p][0], OpSum()), t1 = dec_quad(st[p][1], OpSum());
+        x[8] = lq < 2 ? (lq ? t1 : t0) * 0.125f : -INFINITY;
+        float mx = x[0], sum = 0.0f;
+#pragma unroll
+        for (int i = 1; i < 9; i++) mx = fmaxf(mx, x[i]);
+        mx = dec_quad(mx, OpMax());
+#pragma unroll
+        for (int i = 0; i < 9; i++) { x[i] = exp_fast(x[i] - mx); sum += x[i]; }
+        sum = dec_quad(sum, OpSum());
         const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-        const int row = 4 * lq + v;
-        P[row * DA_PS + lr] = x0 * inv;
-        P[row * DA_PS + 16 + lr] = x1 * inv;
-        P[row * DA_PS + 32 + lr] = x2 * inv;
+#pragma unroll
+        for (int i = 0; i < 9; i++) D[i] = p ? D[i] - x[i] * inv : x[i] * inv;
     }
-    /* v in LDS: this wave's transfers done (vmcnt), then the barrier publishes every wave's
-     * (and orders each wave's P stores before its reads below) */
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
 
-    /* O = P v over keys 12 lq + s (keys >= 34 have P = 0 and multiply zero v) */
     f32x4_dec oc[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) oc[j] = f32x4_dec{0.0f, 0.0f, 0.0f, 0.0f};
-    {
-        float pf[12];
 #pragma unroll
-        for (int c4 = 0; c4 < 3; c4++) {
-            const float4 p4 = *reinterpret_cast<const float4 *>(&P[lr * DA_PS + lq * 12 + 4 * c4]);
-            pf[4 * c4 + 0] = p4.x; pf[4 * c4 + 1] = p4.y; pf[4 * c4 + 2] = p4.z; pf[4 * c4 + 3] = p4.w;
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < 12; s2++) {
-            const int key = lq * 12 + s2;
-            const float4 v4 = Vs[min(key, DEC_S - 1) * 16 + lr];
-            const bool kv = key < DEC_S;
-            const float vf[4] = {kv ? v4.x : 0.0f, kv ? v4.y : 0.0f, kv ? v4.z : 0.0f, kv ? v4.w : 0.0f};
-#pragma unroll
-            for (int j = 0; j < 4; j++) oc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[s2], vf[j], oc[j], 0, 0, 0);
-        }
+    for (int i = 0; i < 9; i++) {
+        const int R = 2 * DEC_S + (i < 8 ? 16 * (i >> 2) + 4 * lq + (i & 3) : 32 + min(lq, 1));
+        const float4 v = sm[R * 16 + ((lr ^ R) & 15)];
+        oc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, D[i], oc[0], 0, 0, 0);
+        oc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, D[i], oc[1], 0, 0, 0);
+        oc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, D[i], oc[2], 0, 0, 0);
+        oc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, D[i], oc[3], 0, 0, 0);
     }
-    /* every product done before the pair-1 waves' O overwrites v and P */
-    __syncthreads();
-    float *Os = sm + qi * (16 * 64);
-    if (pair == 1) {
+    if (qrow < DEC_S) {
+        uint4 *dst = reinterpret_cast<uint4 *>(a.merged + ((size_t)ch * DEC_S + qrow) * DEC_D + h * DEC_HD + 16 * lq);
+        uint32_t w[8];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int v = 0; v < 4; v++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) Os[(j * 4 + v) * 64 + lane] = oc[j][v];
-    }
-    __syncthreads();
-    if (pair == 0) {
-        uint2 *dst = reinterpret_cast<uint2 *>(a.merged + (size_t)ch * DEC_S * DEC_D + h * DEC_HD + 4 * lr);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = qi * 16 + 4 * lq + v;
-            if (row < DEC_S) {
-                uint32_t hv[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) hv[j] = f2h_bits(oc[j][v] - Os[(j * 4 + v) * 64 + lane]);
-                dst[(size_t)row * (DEC_D / 4)] = make_uint2(hv[0] | (hv[1] << 16), hv[2] | (hv[3] << 16));
+            for (int j = 0; j < 4; j += 2) {
+                /* a value that is not finite is NaN, as the difference of two such products is */
+                const float o0 = oc[j][v], o1 = oc[j + 1][v];
+                w[2 * v + j / 2] = (uint32_t)f2h_bits(o0 + (o0 - o0)) | ((uint32_t)f2h_bits(o1 + (o1 - o1)) << 16);
             }
-        }
+        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
     }
 }
 
