@@ -210,13 +210,13 @@ __device__ __forceinline__ uint32_t pack2h_rn(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2_v));
 }
 
-/* QW (3 to 6; KS = 4: 1 or 2) waves of 32 queries per key slice. KS = 1: all keys. KS = 2: 2 QW waves; waves QW..2 QW - 1
+/* QW (3 to 6; KS = 4: 1 to 3) waves of 32 queries per key slice. KS = 1: all keys. KS = 2: 2 QW waves; waves QW..2 QW - 1
  * take the second half of the key tiles with their own LDS buffers, and the halves merge
  * (max, row sum, O) through LDS at the end: twice the waves per query block without any
  * exchange between workgroups. KS = 4: four slices likewise, merged by all waves. Every slice
  * runs the same number of loop trips, so every barrier is reached by all waves. */
 template <int KS, int QW, bool ONE = false>
-__global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS > 2 ? 2 : 4))) void k_flash_attn(AttnArgs a) {
+__global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS == 2 || KS == 1 ? 4 : QW <= 2 ? 2 : 3))) void k_flash_attn(AttnArgs a) {
     /* tile buffers, each [half][KT x 64] fp16, as four separate LDS objects: K and V tiles
      * arrive by LDS DMA (global_load_lds), whose writes count on vmcnt, and the compiler only
      * omits a vmcnt wait before a fragment read when the read provably targets another object
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
     __shared__ __attribute__((aligned(16))) uint16_t Vb0s[KS * KT * 64];
     __shared__ __attribute__((aligned(16))) uint16_t Vb1s[SECOND];
 
-    static_assert(KS > 2 ? QW <= 2 && 8 % KS == 0 : !ONE && QW >= 3 && QW <= 6, "query waves per key slice");
+    static_assert(KS > 2 ? QW <= 3 && 8 % KS == 0 : !ONE && QW >= 3 && QW <= 6, "query waves per key slice");
     /* the wave index in a scalar register: everything derived from it stays scalar */
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int half = KS == 1 ? 0 : wid / QW;
@@ -428,14 +428,18 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
          * barrier), and slice h finishes 8 / KS of the groups of its query wave. A slice without
          * keys has the starting m and l = O = 0: weight zero (slice 0 always has keys). */
         __shared__ __attribute__((aligned(16))) float lm[2 * KS * QW * 64];
-        static_assert(KS * KT * 64 * 2 >= KS * QW * 4 * 64 * 16, "the O groups fit the tile buffers");
-        float4 *const x0 = reinterpret_cast<float4 *>(Kb0s), *const x1 = reinterpret_cast<float4 *>(Vb0s);
+        constexpr int GB = QW <= 2 || ONE ? 4 : 2;   /* groups of one dt in a buffer: four, or two each in the first and second */
+        static_assert(KS * KT * 64 * 2 >= KS * QW * GB * 64 * 16, "the O groups fit the tile buffers");
+        auto xg = [&](int dt, int rq, int slot) __attribute__((always_inline)) -> float4 * {
+            uint16_t *b = rq < GB ? (dt ? Vb0s : Kb0s) : (dt ? Vb1s : Kb1s);
+            return reinterpret_cast<float4 *>(b) + (slot * GB + rq % GB) * 64 + lane;
+        };
         const int slot = half * QW + wave;
 #pragma unroll
-        for (int rq = 0; rq < 4; rq++) {
-            x0[(slot * 4 + rq) * 64 + lane] = make_float4(oacc[0][4 * rq], oacc[0][4 * rq + 1], oacc[0][4 * rq + 2], oacc[0][4 * rq + 3]);
-            x1[(slot * 4 + rq) * 64 + lane] = make_float4(oacc[1][4 * rq], oacc[1][4 * rq + 1], oacc[1][4 * rq + 2], oacc[1][4 * rq + 3]);
-        }
+        for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++)
+                *xg(dt, rq, slot) = make_float4(oacc[dt][4 * rq], oacc[dt][4 * rq + 1], oacc[dt][4 * rq + 2], oacc[dt][4 * rq + 3]);
         lm[slot * 64 + lane] = lrow;
         lm[(KS * QW + slot) * 64 + lane] = m_use;
         __syncthreads();
@@ -457,11 +461,10 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
 #pragma unroll
         for (int i = 0; i < 8 / KS; i++) {
             const int gr = half * (8 / KS) + i, rq = gr & 3;
-            const float4 *x = gr < 4 ? x0 : x1;
             float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int h = 0; h < KS; h++) {
-                const float4 v = x[((h * QW + wave) * 4 + rq) * 64 + lane];
+                const float4 v = *xg(gr >> 2, rq, h * QW + wave);
                 o = make_float4(o.x + v.x * w[h], o.y + v.y * w[h], o.z + v.z * w[h], o.w + v.w * w[h]);
             }
             const int d = 32 * (gr >> 2) + 8 * rq + 4 * g;
@@ -555,15 +558,22 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
      * ties to 4: the cross attention at S = 1296, 32 heads takes 3 (10.8 -> 10.4 us) */
     const int tiles = (Nk + KT - 1) / KT;
     const bool split = tiles >= 8;
-    /* few queries: the keys in four slices, with one or two query waves each, while that leaves
+    /* few queries: the keys in four slices, with one or two (or three, below) query waves each, while that leaves
      * every CU at most one workgroup. A workgroup then walks a quarter of the key tiles and
      * twice to four times as many CUs work: one sequence of 172 (16 heads, 3 tiles) 5.9 -> 4.6 us,
      * 172 x 256 keys 6.3 -> 4.4, 344 8.3 -> 6.0, two of 512 9.6 -> 7.9, 710 11.6 -> 9.2, 1000 14.7 -> 10.9.
      * Past one workgroup per CU it loses (1296: 17.6 -> 23.6 us), as it does with too few tiles to
      * share (40 keys 4.0 -> 4.3; two query waves on 100 keys 5.2 -> 5.5). Eight slices of one wave
-     * were slower than four at every length up to 512 keys. */
-    const long t1 = (long)((Nq + 31) / 32) * BH, t2 = (long)((Nq + 63) / 64) * BH;
-    const int four = tiles >= 2 && t1 <= 256 ? 1 : tiles >= 3 && t2 <= 256 ? 2 : 0;
+     * were slower than four at every length up to 512 keys.
+     * Three query waves per slice, 12 waves in a workgroup, where those blocks still give every CU
+     * at most one and their waves walk fewer tiles than the two-half form's (3 ceil(t / 4) against
+     * 2 ceil(t / 2) per SIMD, less than that by two or more: 513 and 600 keys gain nothing): two of
+     * 710 11.8 -> 11.1 us, 700 x 1300 keys 17.1 -> 15.7, one of 1100 15.2 -> 13.6, 1296 17.1 -> 15.6, 1500
+     * 18.8 -> 16.6. Not with weights to prefetch: this form leaves no CU idle for them, and the
+     * kernels after it lost more than it gained (a W8A8 step of two 710-token sequences 2296 -> 2358
+     * us). Four query waves per slice were slower than the two-half form (710 12.7 us). */
+    const long t1 = (long)((Nq + 31) / 32) * BH, t2 = (long)((Nq + 63) / 64) * BH, t3 = (long)((Nq + 95) / 96) * BH;
+    const int four = tiles >= 2 && t1 <= 256 ? 1 : tiles >= 3 && t2 <= 256 ? 2 : split && !a.npf && t3 <= 256 && 3 * ((tiles + 3) / 4) + 1 < 2 * ((tiles + 1) / 2) ? 3 : 0;
     int qw = 4;
     if (four) {
         qw = four;
@@ -571,7 +581,7 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
         for (int w = 4; w <= 6; w++)
             if ((long)((Nq + 32 * w - 1) / (32 * w)) * BH <= 256) { qw = w; break; }
     } else {
-        const long t4 = (long)((Nq + 127) / 128) * BH, t3 = (long)((Nq + 95) / 96) * BH;
+        const long t4 = (long)((Nq + 127) / 128) * BH;
         if ((t3 + 255) / 256 * 3 < (t4 + 255) / 256 * 4) qw = 3;
     }
     a.nqb = (Nq + 32 * qw - 1) / (32 * qw);
@@ -591,6 +601,7 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
         const bool one = tiles <= 4;   /* a tile per slice: no second buffers */
         if (four == 1 && one) hipLaunchKernelGGL((k_flash_attn<4, 1, true>), grid, dim3(256), 0, s, a);
         else if (four == 1) hipLaunchKernelGGL((k_flash_attn<4, 1>), grid, dim3(256), 0, s, a);
+        else if (four == 3) hipLaunchKernelGGL((k_flash_attn<4, 3>), grid, dim3(768), 0, s, a);
         else if (one) hipLaunchKernelGGL((k_flash_attn<4, 2, true>), grid, dim3(512), 0, s, a);
         else hipLaunchKernelGGL((k_flash_attn<4, 2>), grid, dim3(512), 0, s, a);
     } else if (split) {

@@ -1,5 +1,5 @@
-"""The attention's four-slice form (k_attn.hip: few queries, the keys shared by four slices of one
-or two query waves) against float64 softmax(q k^T / 8) v of the same fp16 operands.
+"""The attention's four-slice form (k_attn.hip: few queries, the keys shared by four slices of one,
+two or three query waves) against float64 softmax(q k^T / 8) v of the same fp16 operands.
 
 Tolerance: the probabilities are rounded to fp16 (2^-11 of each, or 2^-25 where they are subnormal;
 the largest is at least 1) and divided by the sum of the rounded ones, so both roundings count once
@@ -38,8 +38,9 @@ def _check(got, q, k, v, out_f16):
     assert np.all(np.abs(got - want) <= tol), np.max(np.abs(got - want) / tol)
 
 
-# one query wave per slice (a workgroup per 32 queries fits the CUs), then two (per 64)
-@pytest.mark.parametrize("BH,H,Nq", [(2, 1, 1), (4, 2, 31), (2, 2, 33), (16, 16, 172), (64, 16, 130), (64, 16, 255)])
+# one query wave per slice (a workgroup per 32 queries fits the CUs), two (per 64) and, on 512 and
+# 1000 keys, three (per 96)
+@pytest.mark.parametrize("BH,H,Nq", [(64, 16, 257), (64, 16, 384), (2, 1, 1), (4, 2, 31), (2, 2, 33), (16, 16, 172), (64, 16, 130), (64, 16, 255)])
 @pytest.mark.parametrize("Nk", [65, 128, 129, 172, 256, 257, 512, 513, 1000])
 def test_lengths(hip, BH, H, Nq, Nk):
     r = rng(BH + Nq + Nk)
@@ -48,15 +49,15 @@ def test_lengths(hip, BH, H, Nq, Nk):
         _check(_run(hip, q, k, v, H, out_f16), q, k, v, out_f16)
 
 
-@pytest.mark.parametrize("BH,Nq", [(4, 40), (64, 130)])
-def test_slices_of_keys_that_score_minus_infinity(hip, BH, Nq):
+@pytest.mark.parametrize("BH,Nq,Nk", [(4, 40, 256), (64, 130, 256), (64, 300, 512)])
+def test_slices_of_keys_that_score_minus_infinity(hip, BH, Nq, Nk):
     """The second slice's keys all score -inf: weight zero, as if they were not there. All keys so:
     not a number."""
     r = rng(7)
-    q, k, v = (randn(r, (BH, n, 64)).astype(np.float16) for n in (Nq, 256, 256))
+    q, k, v = (randn(r, (BH, n, 64)).astype(np.float16) for n in (Nq, Nk, Nk))
     q[:, :, 0] = np.abs(q[:, :, 0]) + np.float16(0.5)
-    k[:, 64:128, 0] = -np.inf
-    left = np.r_[0:64, 128:256]
+    k[:, Nk // 4:Nk // 2, 0] = -np.inf
+    left = np.r_[0:Nk // 4, Nk // 2:Nk]
     _check(_run(hip, q, k, v, 4, 0), q, k[:, left], v[:, left], 0)
     k[:, :, 0] = -np.inf
     assert np.isnan(_run(hip, q, k, v, 4, 0)).all()
