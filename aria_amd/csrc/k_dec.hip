@@ -230,16 +230,21 @@ __global__ __launch_bounds__(64 * DA_WAVES) void k_dec_attn_mfma(DecAttnArgs a, 
  * 16 rows of each 17-row group, the trim and aria_unpatch_stereo). Feature position p is seq row
  * (p / 16) * 17 + 1 + p % 16.
  * The reference keeps this product in fp32. The fp32 MFMA runs at a sixteenth of the bf16 rate
- * and bound it (307 us of a 60 s decode, 52 % of that pipe's peak; the im2col before it another 35
- * us), so every fp32 operand is split into three bf16 parts, x = x0 + x1 + x2, each the top eight
- * bits of what the parts before it left: 24 bits in all, so the split is exact. x y is then the six
- * products x_i y_j with i + j <= 2; the three left out are below 2^-23 of x y. x0 y0 has an
+ * and bound it (at T = 646 234 us, and 31 for the im2col before it), so every fp32 operand is split
+ * into three bf16 parts, x = x0 + x1 + x2, each the nearest one to what the parts before it left (the
+ * method of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype for
+ * Higher-Precision Computations", ARITH 2019): 24 bits in all, so the split is exact down to bf16's
+ * last bit, 2^-133. x y is then the six products x_i y_j with i + j <= 2; as |x1| <= 2^-8 |x| and
+ * |x2| <= 2^-17 |x|, the three left out are at most 2^-24 (1 + 2^-10) of x y, of either sign (parts cut
+ * off instead of rounded leave out up to 2^-21, always with the product's sign). x0 y0 has an
  * accumulator of its own and the five small products another, which is added at the end, so the
  * large sum is rounded 144 times (once per MFMA) where the fp32 MFMA rounded it 1152 times.
  * A non-finite operand keeps its class: the parts after x0 are zero, and a sum whose large part is
- * not finite is that part alone. Relative error against float64, T = 1 .. 646 and values scaled by
- * 1e-4 .. 300: 2.1-3.0e-7 where the fp32 MFMA had 6.1-8.6e-7. Time, split included: T = 108 64 -> 37 us,
- * T = 300 140 -> 87 us, T = 646 261 -> 144 us.
+ * not finite is that part alone (also one within 2^-7 of the largest float: x0 y0 can exceed x y).
+ * Relative error against float64, T = 1 .. 646 and values scaled by 1e-4 .. 300: 2.0-2.9e-7 where the
+ * fp32 MFMA had 6.1-8.6e-7; where one product makes up the sum, 1.0e-7 at most (4.7e-7 with parts cut
+ * off). Time alone, the input pass (im2col before, the split now) + the product: T = 108 8 + 56 -> 4 +
+ * 32 us, T = 300 16 + 124 -> 6 + 78, T = 646 31 + 234 -> 13 + 125.
  *
  * Layout: a row of 32-k blocks, 192 bytes each: the three parts of the block's 32 values, 64 bytes
  * a part. Features sit in rows 1 .. of xs (row 0 and the row past the end are the convolution's
@@ -251,6 +256,9 @@ __global__ __launch_bounds__(64 * DA_WAVES) void k_dec_attn_mfma(DecAttnArgs a, 
 #define MAP_XROW (24 * MAP_BB)      /* bytes of a feature row */
 #define MAP_N 512
 
+/* bf16 nearest to the finite value of these bits (ties to even) */
+__device__ __forceinline__ uint32_t bf16_rn(uint32_t u) { return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16; }
+
 /* the three bf16 parts of x, as bits; the remainders are exact in fp32 */
 __device__ __forceinline__ void bf16x3(float x, uint32_t (&p)[3]) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x);
@@ -260,10 +268,11 @@ __device__ __forceinline__ void bf16x3(float x, uint32_t (&p)[3]) {
         if (u & 0x007FFFFFu) p[0] |= 0x0040u;   /* a NaN stays one without its low bits */
         return;
     }
-    const float r = x - __builtin_bit_cast(float, u & 0xFFFF0000u);
-    const uint32_t v = __builtin_bit_cast(uint32_t, r);
-    p[1] = v >> 16;
-    p[2] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, v & 0xFFFF0000u)) >> 16;
+    const uint32_t n = bf16_rn(u);
+    if ((n & 0x7F80u) != 0x7F80u) p[0] = n;     /* a value that would round to infinity stays truncated */
+    const float r = x - __builtin_bit_cast(float, p[0] << 16);
+    p[1] = bf16_rn(__builtin_bit_cast(uint32_t, r));
+    p[2] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, p[1] << 16)) >> 16;
 }
 
 /* eight values -> a 16-byte chunk of each part */

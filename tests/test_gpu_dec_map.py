@@ -1,10 +1,11 @@
 """The decoder's mapping convolution on split operands (k_dec_split, k_dec_split_w, k_dec_map in
 k_dec.hip) against a float64 convolution of the same fp32 values.
 
-Bound: the three bf16 parts hold all 24 bits of a value, and the three part products left out are
-together below 2^-22 of each product. The sums round in fp32: 144 additions of the large part and 720
-of the small parts (2^-8 of it), each by at most 2^-24 of the running sum, which is at most the sum
-of absolute products. Hence |error| <= (2^-22 + 152 * 2^-24) sum |x w| + 2^-23 |result|.
+Bound: the three bf16 parts hold all 24 bits of a value, each rounded to the nearest, and the three
+part products left out are together at most 2^-24 (1 + 2^-10) of each product. The sums round in fp32:
+144 additions of the large part and 720 of the small parts (2^-7 of it), each by at most 2^-24 of the
+running sum, which is at most the sum of absolute products. Hence
+|error| <= (2^-24 + 152 * 2^-24) sum |x w| + 2^-23 |result|.
 """
 from __future__ import annotations
 
@@ -60,10 +61,50 @@ def test_map_matches_float64(hip, T, form):
     x = _columns(seq, T).reshape(16 * T, -1)
     w = W.astype(np.float64)
     want = _audio(x @ w.T + b, T)
-    bound = _audio((2.0 ** -22 + 152 * 2.0 ** -24) * (np.abs(x) @ np.abs(w).T), T) + 2.0 ** -23 * np.abs(want) + 1e-12
+    bound = _audio((2.0 ** -24 + 152 * 2.0 ** -24) * (np.abs(x) @ np.abs(w).T), T) + 2.0 ** -23 * np.abs(want) + 1e-12
     got = _run(hip, seq, W, b, T, form)
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
     assert np.array_equal(_run(hip, seq, W, b, T, form), got)
+
+
+def _low_ones(r, shape, sign):
+    """values whose low 16 mantissa bits are all ones, or one bit around half of them: the remainders of
+    the parts are as large as they get"""
+    m = r.integers(0, 128, shape, np.uint32) << np.uint32(16) | r.choice(np.array([0xFFFF, 0x7FFF, 0x8001, 0xFF7F], np.uint32), shape)
+    v = (m | np.uint32(127 << 23)).view(np.float32)
+    return v if sign is None else v * r.choice(np.array(sign, np.float32), shape)
+
+
+@pytest.mark.parametrize("form", [1, 2, 3])
+@pytest.mark.parametrize("T", [1, 12])
+def test_map_one_product(hip, T, form):
+    """Every output is a single product, so nothing averages out: the products left out (2^-24 of it),
+    the five small ones' roundings (2^-24 of 2^-7 of it each) and the final sum's."""
+    r = rng(80 + T)
+    seq = np.zeros((17 * (T + T % 2), 768), np.float32)
+    seq[np.arange(seq.shape[0]), r.integers(0, 768, seq.shape[0])] = _low_ones(r, seq.shape[0], (1, -1))
+    W = np.zeros((512, 768, 3), np.float32)
+    W[:, :, 1] = _low_ones(r, (512, 768), (1, -1))   # the middle tap: one feature row an output
+    W = W.reshape(512, 2304)
+    b = np.zeros(512, np.float32)
+    want = _audio(_columns(seq, T).reshape(16 * T, -1) @ W.astype(np.float64).T, T)
+    got = _run(hip, seq, W, b, T, form)
+    assert np.all(want != 0)
+    assert np.max(np.abs(got / want - 1)) <= 2.1 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("form", [1, 2, 3])
+def test_map_products_of_one_sign(hip, form):
+    """All products positive, low mantissa bits all ones: what is left out of them adds up."""
+    T = 5
+    r = rng(90)
+    seq = _low_ones(r, (17 * (T + T % 2), 768), None)
+    W, b = _low_ones(r, (512, 2304), None), np.zeros(512, np.float32)
+    x, w = _columns(seq, T).reshape(16 * T, -1), W.astype(np.float64)
+    want = _audio(x @ w.T, T)
+    got = _run(hip, seq, W, b, T, form)
+    bound = (153 * 2.0 ** -24 + 2.0 ** -23) * want
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
 
 
 @pytest.mark.parametrize("form", [1, 2, 3])
