@@ -155,6 +155,10 @@ hipError_t aria_k_qgemm_t(void *y, int y_f16, const void *x, int x_f16, int wtyp
  * pass that stages them as fp16 first; both give the same rounded operands */
 int aria_k_qgemm_f32_direct(const void *y, int y_f16, const void *x, int wtype, const void *q,
                             const float *scale, const float *bias, int M, int K, int N);
+/* the kernel that fp16 activations of these arguments take (tiles 0, no epilogue): a k_qgemm_big.hip
+ * configuration, 100 + a k_qgemm_ks.hip one, or -1 for the other kernels */
+int aria_k_qgemm_route(const void *y, int y_f16, const void *x, int wtype, const void *q, const float *scale,
+                       const float *bias, int M, int K, int N);
 /* the same with a fused epilogue (epi NULL = STORE); HEADS needs N % 64 == 0 */
 hipError_t aria_k_qgemm_e(void *y, int y_f16, const void *x, int x_f16, int wtype, const void *q,
                           const float *scale, const float *bias, int M, int K, int N, int tiles,

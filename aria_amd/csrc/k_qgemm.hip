@@ -453,6 +453,12 @@ static bool qgemm_aligned(const QArgs &a, int wt) {
            (wt != ARIA_WQ8 || ((uintptr_t)a.scale & 15u) == 0) && (wt != ARIA_WQ4 || ((uintptr_t)a.scale & 7u) == 0);
 }
 
+/* the output and the activations (xb bytes each) share memory */
+static bool qgemm_overlaps(const QArgs &a, int xb) {
+    const uintptr_t x0 = (uintptr_t)a.x, y0 = (uintptr_t)a.y;
+    return x0 < y0 + (size_t)a.M * a.N * (a.y_f16 ? 2 : 4) && y0 < x0 + (size_t)a.M * a.K * xb;
+}
+
 /* fp32 activations straight into the K-split kernel: its configuration (the first of 32 x 32, 32 x 64
  * and 64 x 64 whose tiles fit one round of the 256 CUs), or -1. It reads twice the activation bytes
  * per tile, and saves the staging pass (a launch of 3 us and one more dependent kernel) or, where
@@ -466,8 +472,7 @@ static bool qgemm_aligned(const QArgs &a, int wt) {
  * workgroup store rows that another has yet to read. */
 static int qgemm_f32_pick(const QArgs &a, int wt) {
     if (a.K % 64 || a.K > 2048 || !qgemm_aligned(a, wt) || (wt == ARIA_WQ4 && ((uintptr_t)a.scale & 15u))) return -1;
-    const uintptr_t x0 = (uintptr_t)a.x, y0 = (uintptr_t)a.y;
-    if (x0 < y0 + (size_t)a.M * a.N * (a.y_f16 ? 2 : 4) && y0 < x0 + (size_t)a.M * a.K * 4) return -1;
+    if (qgemm_overlaps(a, 4)) return -1;
     const long long m32 = (a.M + 31) / 32, m64 = (a.M + 63) / 64, n32 = (a.N + 31) / 32, n64 = (a.N + 63) / 64;
     return m32 * n32 <= 256 ? 0 : m32 * n64 <= 256 ? 1 : m64 * n64 <= 256 ? 2 : -1;
 }
@@ -478,6 +483,42 @@ extern "C" int aria_k_qgemm_f32_direct(const void *y, int y_f16, const void *x, 
     memset(&a, 0, sizeof a);
     a.y = (void *)y; a.y_f16 = y_f16; a.x = x; a.q = q; a.scale = scale; a.bias = bias; a.M = M; a.K = K; a.N = N;
     return qgemm_f32_pick(a, wtype) >= 0;
+}
+
+/* The kernel for fp16 activations with no tile asked for: a k_qgemm_big.hip configuration, GEMM_KS + a
+ * k_qgemm_ks.hip one, or -1 (the kernels below). The k_qgemm_big.hip configurations at M = 2592, from
+ * which qgemm_pick starts: N <= 1024 without HEADS (96 x 128
+ * tiles, two workgroups per CU), HEADS with N <= 3072 (the qkv projection: 64 x 512 in
+ * 8-wave workgroups, one per CU), other N <= 3072 without HEADS (128 x 128, two per CU), N = 4096
+ * (192 x 256 in 8-wave workgroups, one per CU) and wider (224 x 128); N <= 1024 with an
+ * even number of K-tiles in 96 x 128
+ * tiles of 8 waves, the two halves of K on their own pipelines (216 tiles at M = 2592
+ * leave 40 CUs idle; the split doubles the waves on the busy ones), and HEADS with N <=
+ * 1024 (ca_q) likewise in 64 x 256 tiles (164 tiles: one workgroup per busy CU, so the
+ * split's second half is what gives those CUs two waves per SIMD; 15.6 -> 15.2 us);
+ * HEADS wider than 3072 stays on the weights-in-registers kernel. fp16 weights: qgemm_big_f16_pick's,
+ * and for HEADS, which needs 64 columns per wave, the LDS-operand kernel where qgemm_pick finds none.
+ * An output over the activations (fp16, in place: K = N) keeps them: up to N = 128 a tile has whole
+ * rows there, read to the end before the first is stored, where one of several narrower tiles would
+ * store what the next has yet to read. */
+static int qgemm_route(const QArgs &a, int wt) {
+    if (a.K % 64 || (a.gelu && a.epi.mode != ARIA_EPI_STORE) || (wt == ARIA_WQ4 && ((uintptr_t)a.scale & 15u))) return -1;
+    const bool heads = a.epi.mode == ARIA_EPI_HEADS, even = (a.K / 64) % 2 == 0;
+    const int cur = wt == ARIA_WF16 ? (heads ? -1 : qgemm_big_f16_pick(a.M, a.N))
+                  : heads ? (a.N <= 1024 && even ? 6 : a.N <= 3072 ? 8 : -1)
+                  : a.N <= 1024 ? (even ? 5 : 0) : a.N <= 3072 ? 1 : a.N <= 4096 ? 7 : 4;
+    if (cur < 0 && wt != ARIA_WF16) return -1;
+    if (a.epi.mode == ARIA_EPI_STORE && qgemm_overlaps(a, 2)) return cur;
+    return qgemm_pick(wt, heads, a.M, a.N, a.K, cur);
+}
+
+extern "C" int aria_k_qgemm_route(const void *y, int y_f16, const void *x, int wtype, const void *q, const float *scale,
+                                  const float *bias, int M, int K, int N) {
+    QArgs a;
+    memset(&a, 0, sizeof a);
+    a.y = (void *)y; a.y_f16 = y_f16; a.x = x; a.q = q; a.scale = scale; a.bias = bias; a.M = M; a.K = K; a.N = N;
+    a.epi.mode = ARIA_EPI_STORE;
+    return qgemm_aligned(a, wtype) ? qgemm_route(a, wtype) : -1;
 }
 
 template <int WT, bool AF16>
@@ -498,41 +539,13 @@ static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
         return hipGetLastError();
     } else {
     if (tiles >= GEMM_KS) return qgemm_ks_launch(a, WT, tiles - GEMM_KS, s);   /* explicit: configuration tiles - GEMM_KS */
-    if constexpr (WT == ARIA_WF16) {
-        /* fp16 weights on the LDS-DMA kernel: explicit tiles 13.., or the configuration that
-         * qgemm_big_f16_pick chooses for the shape (HEADS, which needs 64 columns per wave,
-         * stays on the LDS-operand kernel) */
-        if (tiles >= 13) return qgemm_big_launch(a, WT, tiles - 13, s);
-        if (tiles == 0 && a.K % 64 == 0 && (!a.gelu || a.epi.mode == ARIA_EPI_STORE)) {
-            const bool heads = a.epi.mode == ARIA_EPI_HEADS;
-            const int c = qgemm_pick(WT, heads, a.M, a.N, a.K, heads ? -1 : qgemm_big_f16_pick(a.M, a.N));
-            if (c >= GEMM_KS) return qgemm_ks_launch(a, WT, c - GEMM_KS, s);
-            if (c >= 0) return qgemm_big_launch(a, WT, c, s);
-        }
+    if (tiles >= 13) return qgemm_big_launch(a, WT, tiles - 13, s);   /* likewise: k_qgemm_big.hip's tiles - 13 */
+    if (tiles == 0) {
+        const int c = qgemm_route(a, WT);
+        if (c >= GEMM_KS) return qgemm_ks_launch(a, WT, c - GEMM_KS, s);
+        if (c >= 0) return qgemm_big_launch(a, WT, c, s);
     }
     if constexpr (WT != ARIA_WF16) {
-        /* the LDS-DMA kernel (k_qgemm_big.hip): explicit tiles 13.. (configuration tiles - 13),
-         * or its configuration at M = 2592, from which qgemm_pick starts: N <= 1024 without HEADS (96 x 128
-         * tiles, two workgroups per CU), HEADS with N <= 3072 (the qkv projection: 64 x 512 in
-         * 8-wave workgroups, one per CU), other N <= 3072 without HEADS (128 x 128, two per CU), N = 4096
-         * (192 x 256 in 8-wave workgroups, one per CU) and wider (224 x 128); N <= 1024 with an
-         * even number of K-tiles in 96 x 128
-         * tiles of 8 waves, the two halves of K on their own pipelines (216 tiles at M = 2592
-         * leave 40 CUs idle; the split doubles the waves on the busy ones), and HEADS with N <=
-         * 1024 (ca_q) likewise in 64 x 256 tiles (164 tiles: one workgroup per busy CU, so the
-         * split's second half is what gives those CUs two waves per SIMD; 15.6 -> 15.2 us);
-         * HEADS wider than 3072 stays on the weights-in-registers kernel */
-        if (tiles >= 13) return qgemm_big_launch(a, WT, tiles - 13, s);
-        if (tiles == 0 && a.K % 64 == 0 && (WT != ARIA_WQ4 || ((uintptr_t)a.scale & 15u) == 0) &&
-            (!a.gelu || a.epi.mode == ARIA_EPI_STORE)) {
-            const bool heads = a.epi.mode == ARIA_EPI_HEADS;
-            const int cfg = heads ? (a.N <= 1024 && (a.K / 64) % 2 == 0 ? 6 : a.N <= 3072 ? 8 : -1)
-                          : a.N <= 1024 ? ((a.K / 64) % 2 == 0 ? 5 : 0) : a.N <= 3072 ? 1 : a.N <= 4096 ? 7 : 4;
-            if (cfg >= 0) {
-                const int c = qgemm_pick(WT, heads, a.M, a.N, a.K, cfg);
-                return c >= GEMM_KS ? qgemm_ks_launch(a, WT, c - GEMM_KS, s) : qgemm_big_launch(a, WT, c, s);
-            }
-        }
         /* weights-in-registers kernel: explicit tiles 9..12 (BM = 32 * (tiles - 8)), or the pick */
         int fm = (tiles > NCFG) ? tiles - NCFG : (tiles == 0 ? pick_wr(a.M, a.N, a.K) : 0);
         /* Q8 with N and K <= 1024 (the DiT's sa_out / ca_out): 64 x 64 LDS-operand tiles, 2.5

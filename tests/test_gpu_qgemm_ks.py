@@ -205,3 +205,42 @@ def test_pick_names_a_kernel_that_takes_the_shape():
             assert c not in halves or even
             assert not heads or c in ((1, 5) if wt == I8 else (6, 8))
     assert {c for _, _, c in seen} >= {KS + i for i in range(5)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wt", [Q8, Q4, F16])
+def test_in_place(hip, port, wt):
+    """fp16 activations overwritten by the output (K = N, one column tile): as with an output of its own."""
+    from aria_amd.device import DeviceArray
+    L = hip.lib()
+    for M, K in ((33, 64), (172, 128), (1000, 64), (2592, 128)):
+        op = Op(hip, port, wt, M, K, K, 900 + wt)
+        x = op.dx.to_host()
+        for fn in ("aria_hip_qlinear_dev", "aria_hip_qlinear_noalloc_dev"):
+            d = DeviceArray.from_host(x)
+            hip.check(getattr(L, fn)(d.p, 1, d.p, 1, wt, op.dq.p, op.ds.p if op.ds else None, op.db.p, M, K, K, None))
+            hip.check(L.aria_hip_stream_sync(None))
+            bound = op.bound + 2.0 ** -11 * np.abs(op.want) + 2.0 ** -25
+            assert np.all(np.abs(d.to_host() - op.want) <= bound), (M, K, fn)
+
+
+def test_route_keeps_whole_rows_in_place():
+    """An output that overlaps fp16 activations never takes the K-split kernel's narrow tiles, which
+    others take at these sizes; one that only touches them does."""
+    import aria_amd
+    try:
+        f = aria_amd.lib().aria_k_qgemm_route
+    except (aria_amd.HipError, OSError) as e:
+        pytest.skip(f"library not built: {e}")
+    f.restype = C.c_int
+    f.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p, C.c_int] + [C.c_void_p] * 3 + [C.c_int] * 3
+    base = 1 << 40   # addresses only compared
+    x, y, q, s, b = (base + (i << 36) for i in range(5))
+    for wt in (Q8, Q4, F16):
+        for K in (64, 128):
+            for M in (1, 33, 172, 710, 2592):
+                assert f(y, 1, x, wt, q, s, b, M, K, K) >= KS
+                assert f(x + 2 * M * K, 1, x, wt, q, s, b, M, K, K) >= KS
+                assert f(x - 2 * M * K, 1, x, wt, q, s, b, M, K, K) >= KS
+                for o in (0, 16, -16, 2 * M * K - 16, 16 - 2 * M * K):
+                    assert 0 <= f(x + o, 1, x, wt, q, s, b, M, K, K) < KS, (wt, K, M, o)
