@@ -200,9 +200,15 @@ typedef struct {
     size_t bytes[ARIA_PF_SPANS];
     int n;
 } aria_prefetch_set;
-/* aria_k_flash_attn that also prefetches pf (NULL: none) on the CUs the split form leaves idle */
+/* aria_k_flash_attn of a block's self-attention: pf is read on the CUs that the launch leaves idle,
+ * and ignored where those are too few. A launch with pf (also one without spans) keeps CUs free for
+ * it, so its form can differ from aria_k_flash_attn's at the same sizes, and with it the order of the
+ * sums; what the spans hold changes nothing. pf NULL: aria_k_flash_attn */
 hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k, const uint16_t *v, void *o, int o_f16,
                                 int BH, int H, int Nq, int Nk, const aria_prefetch_set *pf, hipStream_t s);
+/* how such a launch is shared out on ncu CUs (block: pf given, spans: with something to prefetch):
+ * out = key slices, query waves per slice, workgroups, prefetch workgroups */
+void aria_k_flash_attn_plan(int BH, int Nq, int Nk, int block, int spans, int ncu, int *out);
 
 /* fp32 SIMT GEMM (k_sgemm.hip), batched with element strides sA/sB/sC:
  * C_b[M,N] = alpha * (A_b[M,K] op(B_b)) (+ bias[N]); op(B) = B^T for B_b [N,K]

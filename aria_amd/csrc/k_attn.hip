@@ -532,22 +532,13 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(KS
     }
 }
 
-extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k, const uint16_t *v, void *o,
-                                           int o_f16, int BH, int H, int Nq, int Nk, const aria_prefetch_set *pf,
-                                           hipStream_t s) {
-    if (BH <= 0 || Nq <= 0) return hipSuccess;
-    AttnArgs a;
-    a.npf = 0;
-    if (pf && (pf->n < 0 || pf->n > ARIA_PF_SPANS)) return hipErrorInvalidValue;
-    for (int i = 0; pf && i < pf->n; i++) {
-        if (!pf->p[i] || !pf->bytes[i]) continue;
-        if ((pf->bytes[i] & 15u) || ((uintptr_t)pf->p[i] & 15u) || pf->bytes[i] / 16 > 0xFFFFFFFFu)
-            return hipErrorInvalidValue;
-        a.pf[a.npf] = (const uint4 *)pf->p[i];
-        a.pf_n16[a.npf++] = (unsigned)(pf->bytes[i] / 16);
-    }
-    a.q = q; a.k = k; a.v = v; a.o = o; a.H = H; a.Nq = Nq; a.Nk = Nk; a.o_f16 = o_f16;
-    a.scale_log2 = 0.125f * ARIA_LOG2E;
+/* How a launch is shared out: ks key slices of qw query waves in a workgroup, T workgroups of nqb per
+ * (batch, head), and npw more workgroups that prefetch. The form depends on the sizes and on whether
+ * the call is a block's self-attention (`block`), npw also on whether there is anything to prefetch:
+ * a block gives the same bits by itself and inside a step. */
+struct AttnPlan { int ks, qw, nqb, T, Tpad, npw; };
+static AttnPlan attn_plan(int BH, int Nq, int Nk, bool block, bool spans, int ncu) {
+    AttnPlan p;
     /* split the keys inside the workgroup when there are enough tiles for both halves
      * (S = 1296 self-attention: 21 tiles); short key sets (the 256 cross keys) run one half.
      * A CU running two workgroups takes nearly twice as long as one running a single one, so
@@ -569,46 +560,81 @@ extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k,
      * at most one and their waves walk fewer tiles than the two-half form's (3 ceil(t / 4) against
      * 2 ceil(t / 2) per SIMD, less than that by two or more: 513 and 600 keys gain nothing): two of
      * 710 11.8 -> 11.1 us, 700 x 1300 keys 17.1 -> 15.7, one of 1100 15.2 -> 13.6, 1296 17.1 -> 15.6, 1500
-     * 18.8 -> 16.6. Not with weights to prefetch: this form leaves no CU idle for them, and the
-     * kernels after it lost more than it gained (a W8A8 step of two 710-token sequences 2296 -> 2358
-     * us). Four query waves per slice were slower than the two-half form (710 12.7 us). */
+     * 18.8 -> 16.6. Not in a block: this form leaves no CU idle for the next block's weights, and
+     * the kernels after it lost more than it gained (a W8A8 step of two 710-token sequences 2296 ->
+     * 2358 us). Four query waves per slice were slower than the two-half form (710 12.7 us). */
     const long t1 = (long)((Nq + 31) / 32) * BH, t2 = (long)((Nq + 63) / 64) * BH, t3 = (long)((Nq + 95) / 96) * BH;
-    const int four = tiles >= 2 && t1 <= 256 ? 1 : tiles >= 3 && t2 <= 256 ? 2 : split && !a.npf && t3 <= 256 && 3 * ((tiles + 3) / 4) + 1 < 2 * ((tiles + 1) / 2) ? 3 : 0;
-    int qw = 4;
+    const int four = tiles >= 2 && t1 <= 256 ? 1 : tiles >= 3 && t2 <= 256 ? 2
+                   : split && !block && t3 <= 256 && 3 * ((tiles + 3) / 4) + 1 < 2 * ((tiles + 1) / 2) ? 3 : 0;
+    p.ks = four ? 4 : split ? 2 : 1;
+    p.qw = 4;
     if (four) {
-        qw = four;
+        p.qw = four;
     } else if (split) {
         for (int w = 4; w <= 6; w++)
-            if ((long)((Nq + 32 * w - 1) / (32 * w)) * BH <= 256) { qw = w; break; }
+            if ((long)((Nq + 32 * w - 1) / (32 * w)) * BH <= 256) { p.qw = w; break; }
     } else {
         const long t4 = (long)((Nq + 127) / 128) * BH;
-        if ((t3 + 255) / 256 * 3 < (t4 + 255) / 256 * 4) qw = 3;
+        if ((t3 + 255) / 256 * 3 < (t4 + 255) / 256 * 4) p.qw = 3;
     }
-    a.nqb = (Nq + 32 * qw - 1) / (32 * qw);
-    a.T = a.nqb * BH;
-    a.Tpad = (a.T + 7) / 8 * 8;
-    /* prefetch workgroups on the CUs the split form's one-per-CU workgroups leave idle */
+    p.nqb = (Nq + 32 * p.qw - 1) / (32 * p.qw);
+    p.T = p.nqb * BH;
+    p.Tpad = (p.T + 7) / 8 * 8;
+    /* prefetch workgroups on the CUs that one workgroup per CU leaves idle: of the two-half form, and of the
+     * four-slice forms with eight key tiles or more where they are three eighths of the CUs (fewer read
+     * 10-16 MB for longer than the attention runs). A step of one sequence, without / with, us: 564
+     * tokens (112 idle) q4 2271 / 2193, q8 2213 / 2134, W8A8 2123 / 2097; 604 (96) q4 2223 / 2198, q8 2183 /
+     * 2144, W8A8 2137 / 2120; 664 (80) q4 2243 / 2300, q8 2255 / 2258, W8A8 2236 / 2225; 710 (64) q4 2329 /
+     * 2360, q8 2269 / 2312, W8A8 2251 / 2244; 864 (32) q4 2421 / 2459, W8A8 2315 / 2408; 450 (16) q4 1762 / 2334 */
+    const int idle = ncu - p.Tpad;
+    const bool room = p.ks == 2 ? idle > 0 : p.ks == 4 && split && idle >= 96;
+    p.npw = block && spans && room ? idle / 8 * 8 : 0;
+    return p;
+}
+
+extern "C" void aria_k_flash_attn_plan(int BH, int Nq, int Nk, int block, int spans, int ncu, int *out) {
+    const AttnPlan p = attn_plan(BH, Nq, Nk, block != 0, spans != 0, ncu);
+    out[0] = p.ks; out[1] = p.qw; out[2] = p.T; out[3] = p.npw;
+}
+
+extern "C" hipError_t aria_k_flash_attn_pf(const uint16_t *q, const uint16_t *k, const uint16_t *v, void *o,
+                                           int o_f16, int BH, int H, int Nq, int Nk, const aria_prefetch_set *pf,
+                                           hipStream_t s) {
+    if (BH <= 0 || Nq <= 0) return hipSuccess;
+    AttnArgs a;
+    a.npf = 0;
+    if (pf && (pf->n < 0 || pf->n > ARIA_PF_SPANS)) return hipErrorInvalidValue;
+    for (int i = 0; pf && i < pf->n; i++) {
+        if (!pf->p[i] || !pf->bytes[i]) continue;
+        if ((pf->bytes[i] & 15u) || ((uintptr_t)pf->p[i] & 15u) || pf->bytes[i] / 16 > 0xFFFFFFFFu)
+            return hipErrorInvalidValue;
+        a.pf[a.npf] = (const uint4 *)pf->p[i];
+        a.pf_n16[a.npf++] = (unsigned)(pf->bytes[i] / 16);
+    }
+    a.q = q; a.k = k; a.v = v; a.o = o; a.H = H; a.Nq = Nq; a.Nk = Nk; a.o_f16 = o_f16;
+    a.scale_log2 = 0.125f * ARIA_LOG2E;
     static int ncu = 0;
     if (!ncu) {
         int dev = 0, n = 0;
         ncu = (hipGetDevice(&dev) == hipSuccess &&
                hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : -1;
     }
-    const int npw = (split && !four && a.npf && ncu > a.Tpad) ? (ncu - a.Tpad) / 8 * 8 : 0;
-    if (!npw) a.npf = 0;
-    const dim3 grid(a.Tpad + npw);
-    if (four) {
-        const bool one = tiles <= 4;   /* a tile per slice: no second buffers */
-        if (four == 1 && one) hipLaunchKernelGGL((k_flash_attn<4, 1, true>), grid, dim3(256), 0, s, a);
-        else if (four == 1) hipLaunchKernelGGL((k_flash_attn<4, 1>), grid, dim3(256), 0, s, a);
-        else if (four == 3) hipLaunchKernelGGL((k_flash_attn<4, 3>), grid, dim3(768), 0, s, a);
+    const AttnPlan p = attn_plan(BH, Nq, Nk, pf != nullptr, a.npf > 0, ncu);
+    a.nqb = p.nqb; a.T = p.T; a.Tpad = p.Tpad;
+    if (!p.npw) a.npf = 0;
+    const dim3 grid(p.Tpad + p.npw);
+    if (p.ks == 4) {
+        const bool one = Nk <= 4 * KT;   /* a tile per slice: no second buffers */
+        if (p.qw == 1 && one) hipLaunchKernelGGL((k_flash_attn<4, 1, true>), grid, dim3(256), 0, s, a);
+        else if (p.qw == 1) hipLaunchKernelGGL((k_flash_attn<4, 1>), grid, dim3(256), 0, s, a);
+        else if (p.qw == 3) hipLaunchKernelGGL((k_flash_attn<4, 3>), grid, dim3(768), 0, s, a);
         else if (one) hipLaunchKernelGGL((k_flash_attn<4, 2, true>), grid, dim3(512), 0, s, a);
         else hipLaunchKernelGGL((k_flash_attn<4, 2>), grid, dim3(512), 0, s, a);
-    } else if (split) {
-        if (qw == 6) hipLaunchKernelGGL((k_flash_attn<2, 6>), grid, dim3(768), 0, s, a);
-        else if (qw == 5) hipLaunchKernelGGL((k_flash_attn<2, 5>), grid, dim3(640), 0, s, a);
+    } else if (p.ks == 2) {
+        if (p.qw == 6) hipLaunchKernelGGL((k_flash_attn<2, 6>), grid, dim3(768), 0, s, a);
+        else if (p.qw == 5) hipLaunchKernelGGL((k_flash_attn<2, 5>), grid, dim3(640), 0, s, a);
         else hipLaunchKernelGGL((k_flash_attn<2, 4>), grid, dim3(512), 0, s, a);
-    } else if (qw == 3) {
+    } else if (p.qw == 3) {
         hipLaunchKernelGGL((k_flash_attn<1, 3>), grid, dim3(192), 0, s, a);
     } else {
         hipLaunchKernelGGL((k_flash_attn<1, 4>), grid, dim3(256), 0, s, a);
