@@ -381,8 +381,8 @@ static int pick_wr(int M, int N, int K) {
     return best;
 }
 
-/* ---- which kernel and tile: a launch costs about c0 + n (c1 + ck K / 1024) us, n = the tiles on
- * the busiest of the 256 CUs. The constants are least-squares fits per configuration to a sweep of
+/* ---- which kernel and tile: a launch costs about c0 + n (c1 + ck K / 1024) + co M N / 10^6 us, n = the
+ * tiles on the busiest of the 256 CUs (co, the output's bytes, only in the second set below). The constants are least-squares fits per configuration to a sweep of
  * M = 40 .. 2592 over the DiT's projections (N / K = 1024 / 1024, 3072 / 1024, 4096 / 1024,
  * 8192 / 1024, 1024 / 4096), each launch alone in a replayed graph over six operand sets; rms
  * error 5-9 %. A candidate displaces the configuration that M = 2592 takes only where it is
@@ -391,7 +391,7 @@ static int pick_wr(int M, int N, int K) {
  * the fastest of each shape on average (fp16 4 %). Down to two rows of tiles the small tiles of
  * k_qgemm_ks.hip win because they give every CU work; from about M = 860 (N = 8192) to 1420
  * (N = 1024) on, the large tiles' fewer bytes per product do. */
-struct TileCost { int pick, bm, bn; float c0, c1, ck; };
+struct TileCost { int pick, bm, bn; float c0, c1, ck, co; };
 static const TileCost cost_q8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 1.4f}, {GEMM_KS + 1, 32, 64, 1.2f, 1.7f, 2.0f},
     {GEMM_KS + 2, 64, 64, 1.3f, 3.2f, 2.6f}, {GEMM_KS + 3, 96, 64, 2.0f, 3.9f, 3.2f}, {GEMM_KS + 4, 64, 64, 2.9f, 0.6f, 3.4f},
     {0, 96, 128, 2.5f, 3.4f, 5.5f}, {1, 128, 128, 3.2f, 3.8f, 6.5f}, {4, 224, 128, 8.7f, 6.4f, 6.4f},
@@ -407,6 +407,26 @@ static const TileCost cost_i8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 0.8f}, {GEMM_KS
     {GEMM_KS + 2, 64, 64, 0.9f, 3.4f, 1.4f}, {GEMM_KS + 3, 96, 64, 1.4f, 4.1f, 1.9f}, {0, 64, 128, 2.0f, 3.1f, 2.2f},
     {2, 128, 128, 6.0f, 0.2f, 4.9f}, {3, 192, 128, 7.5f, 2.3f, 5.7f}, {4, 96, 128, -0.2f, 6.1f, 3.4f},
     {6, 192, 256, -6.7f, 12.3f, 12.3f}};
+/* The same away from that sweep, M > 2592 or K < 512, fitted to K = 64 .. 8192 (M > 2592) and 64 .. 768, N = 64 ..
+ * 16384, M up to 12000 (rms error 4-12 %): many tiles of few products are bound by their output, and the
+ * constants above took 64 x 64 K-split tiles for them (Q4, M = 8192, K = 128, N = 16384: 117 us as
+ * 224 x 128 tiles, 237 so; int8, M = 8192, K = 1024, N = 8192: 138 us as 192 x 128 tiles, 151 as 128 x
+ * 128). A candidate has to be predicted 6 % faster; the picks are within 1-2 % of the fastest on average
+ * and at most 6 % behind the configuration they displace, 11 % over shapes that were not fitted. Two
+ * K-split tiles stay out above M = 2592: 96 x 64 (Q8, M = 5184, K = 1024, N = 256 10.2 -> 12.1 us), and
+ * HEADS on any at K < 512 (int8, M = 3000, K = 256, N = 768 8.7 -> 10.5). */
+static const TileCost far_q8[] = {{GEMM_KS, 32, 32, 1.59f, 0.99f, 1.62f, 1.09f}, {GEMM_KS + 1, 32, 64, 1.65f, 1.23f, 2.08f, 0.80f},
+    {GEMM_KS + 2, 64, 64, 1.61f, 1.72f, 3.97f, 0.61f}, {GEMM_KS + 3, 96, 64, 1.44f, 2.37f, 5.61f, 0.49f},
+    {GEMM_KS + 4, 64, 64, 2.78f, 0.29f, 3.99f, 0.61f}, {0, 96, 128, 4.07f, 0.00f, 6.06f, 0.69f}, {1, 128, 128, 4.64f, 0.00f, 7.60f, 0.65f},
+    {4, 224, 128, 6.30f, 0.00f, 11.54f, 0.62f}, {5, 96, 128, 2.33f, 1.60f, 6.63f, 0.82f}, {7, 192, 256, 3.36f, 2.25f, 16.72f, 0.63f}};
+static const TileCost far_q4[] = {{GEMM_KS, 32, 32, 1.68f, 0.97f, 1.79f, 1.36f}, {GEMM_KS + 1, 32, 64, 1.69f, 1.28f, 2.53f, 0.83f},
+    {GEMM_KS + 2, 64, 64, 1.64f, 1.83f, 4.34f, 0.60f}, {GEMM_KS + 3, 96, 64, 1.43f, 2.39f, 5.98f, 0.45f},
+    {GEMM_KS + 4, 64, 64, 2.84f, 0.26f, 4.86f, 0.58f}, {0, 96, 128, 3.91f, 0.00f, 7.52f, 0.61f}, {1, 128, 128, 4.32f, 0.00f, 8.90f, 0.59f},
+    {4, 224, 128, 5.84f, 0.00f, 12.78f, 0.58f}, {5, 96, 128, 2.37f, 1.38f, 8.16f, 0.77f}, {7, 192, 256, 3.38f, 1.83f, 18.52f, 0.63f}};
+static const TileCost far_i8[] = {{GEMM_KS, 32, 32, 1.55f, 1.01f, 0.88f, 1.32f}, {GEMM_KS + 1, 32, 64, 1.67f, 1.22f, 1.18f, 1.03f},
+    {GEMM_KS + 2, 64, 64, 1.74f, 1.80f, 2.04f, 0.83f}, {GEMM_KS + 3, 96, 64, 1.78f, 2.20f, 2.94f, 0.75f},
+    {0, 64, 128, 3.04f, 0.33f, 2.84f, 0.64f}, {2, 128, 128, 4.52f, 0.00f, 4.31f, 0.69f}, {3, 192, 128, 5.72f, 0.00f, 5.56f, 0.63f},
+    {4, 96, 128, 1.87f, 1.91f, 4.07f, 0.74f}, {6, 192, 256, 2.30f, 3.37f, 9.28f, 0.55f}};
 /* HEADS (64 columns in one wave; timed at K = 1024 only, N = 1024 and 3072) */
 static const TileCost cost_q8_heads[] = {{GEMM_KS + 1, 32, 64, 1.1f, 2.4f, 2.0f}, {GEMM_KS + 3, 96, 64, 2.0f, 5.4f, 3.2f},
     {GEMM_KS + 4, 64, 64, 3.5f, 1.2f, 3.4f}, {6, 64, 256, 1.0f, 8.0f, 6.2f}, {8, 64, 512, 7.7f, 6.0f, 9.4f}};
@@ -419,28 +439,30 @@ static const TileCost cost_i8_heads[] = {{GEMM_KS + 1, 32, 64, 0.8f, 2.7f, 1.1f}
 int qgemm_pick(int wt, bool heads, int M, int N, int K, int cur) {
     struct Table { const TileCost *t; int n; };
 #define TBL(x) Table{x, (int)(sizeof x / sizeof x[0])}
-    const Table tb = wt == ARIA_WI8 ? (heads ? TBL(cost_i8_heads) : TBL(cost_i8))
+    const bool far = !heads && wt != ARIA_WF16 && (M > 2592 || K < 512);
+    const Table tb = far ? (wt == ARIA_WI8 ? TBL(far_i8) : wt == ARIA_WQ4 ? TBL(far_q4) : TBL(far_q8))
+                   : wt == ARIA_WI8 ? (heads ? TBL(cost_i8_heads) : TBL(cost_i8))
                    : wt == ARIA_WF16 ? (heads ? TBL(cost_f16_heads) : TBL(cost_f16))
                    : heads ? TBL(cost_q8_heads) : wt == ARIA_WQ4 ? TBL(cost_q4) : TBL(cost_q8);
 #undef TBL
     const float k = (float)K / 1024.0f;
     auto us = [&](const TileCost &c) {
         const long T = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-        return c.c0 + (float)((T + 255) / 256) * (c.c1 + c.ck * k);
+        return c.c0 + (float)((T + 255) / 256) * (c.c1 + c.ck * k) + c.co * ((float)M * (float)N * 1e-6f);
     };
-    /* fp16 HEADS runs on the LDS-operand kernel otherwise: 13.4 us at N = 1024 up to M = 1836, 14 -> 31 us
-     * at N = 3072 from M = 600 to 2592 */
-    float cur_us = wt == ARIA_WF16 && heads ? k * (12.0f + 2.5e-6f * (float)M * (float)N) : 1e30f;
+    /* fp16 HEADS runs on the LDS-operand kernel otherwise: K = 1024 13.4 us at N = 1024 up to M = 1836, 14 ->
+     * 31 us at N = 3072 from M = 600 to 2592; K = 2048, N = 2048 20.4 us at M = 432, 32.4 at M = 1836 */
+    float cur_us = wt == ARIA_WF16 && heads ? 3.4f + k * (8.6f + 2.5e-6f * (float)M * (float)N) : 1e30f;
     for (int i = 0; i < tb.n; i++)
         if (tb.t[i].pick == cur) cur_us = us(tb.t[i]);
     int best = cur;
-    float best_us = 0.92f * cur_us;
+    float best_us = (far ? 0.94f : 0.92f) * cur_us;
     const int steps = K / (wt == ARIA_WI8 ? 128 : 64);
     for (int i = 0; i < tb.n; i++) {
         const TileCost &c = tb.t[i];
         /* only the K-split kernel and the large-tile configurations whose K is unsplit or even */
         const bool split = c.pick < GEMM_KS && (wt == ARIA_WI8 ? c.pick == 4 || c.pick == 5 : wt != ARIA_WF16 && (c.pick == 5 || c.pick == 6));
-        if ((split && steps % 2) || (wt == ARIA_WF16 && c.pick < GEMM_KS)) continue;
+        if ((split && steps % 2) || (wt == ARIA_WF16 && c.pick < GEMM_KS) || (M > 2592 && (heads ? c.pick >= GEMM_KS && K < 512 : far && c.pick == GEMM_KS + 3))) continue;
         const float t = us(c);
         if (t < best_us) { best_us = t; best = c.pick; }
     }

@@ -244,3 +244,25 @@ def test_route_keeps_whole_rows_in_place():
                 assert f(x - 2 * M * K, 1, x, wt, q, s, b, M, K, K) >= KS
                 for o in (0, 16, -16, 2 * M * K - 16, 16 - 2 * M * K):
                     assert 0 <= f(x + o, 1, x, wt, q, s, b, M, K, K) < KS, (wt, K, M, o)
+
+
+# (weight type, HEADS, M, K, N, the configuration that the pick starts from, those measured within 9 % of the
+# fastest): a wide output of few products, more rows than 2592, HEADS at another width, and the DiT's
+MEASURED = ((Q4, 0, 8192, 128, 16384, 4, (1, 3, 4, 7)), (Q8, 0, 5184, 128, 16384, 4, (3, 4, 7)),
+            (Q4, 0, 12000, 256, 4096, 7, (0, 1, 3, 4, 7)), (Q8, 0, 2592, 128, 16384, 4, (0, 1, 3, 4)),
+            (Q4, 0, 1836, 256, 4096, 7, (1, 7, 8)), (Q8, 0, 3500, 4096, 1024, 5, (1, 2, 6)),
+            (Q8, 0, 5184, 1024, 256, 5, (0, 5)), (I8, 0, 8192, 1024, 8192, 3, (3,)), (I8, 0, 5184, 1024, 4096, 6, (3, 6)),
+            (I8, 0, 8192, 1536, 6144, 3, (3,)), (I8, 0, 8192, 4096, 1024, 4, (1, 2)), (F16, 1, 1836, 2048, 2048, -1, (-1,)),
+            (Q8, 0, 172, 4096, 1024, 5, (KS,)), (Q4, 0, 710, 4096, 1024, 5, (KS + 2,)), (Q8, 0, 2592, 1024, 4096, 7, (3, 7)),
+            (F16, 1, 172, 1024, 3072, -1, (KS + 2, KS + 4)))
+
+
+@pytest.mark.parametrize("wt,heads,M,K,N,cur,fast", MEASURED)
+def test_pick_is_among_the_fastest_measured(wt, heads, M, K, N, cur, fast):
+    import aria_amd
+    try:
+        pick = aria_amd.lib()._Z10qgemm_pickibiiii
+    except (aria_amd.HipError, OSError) as e:
+        pytest.skip(f"library not built: {e}")
+    pick.restype, pick.argtypes = C.c_int, [C.c_int, C.c_bool] + [C.c_int] * 4
+    assert pick(wt, bool(heads), M, N, K, cur) in fast
