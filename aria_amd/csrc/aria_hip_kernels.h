@@ -76,9 +76,8 @@ hipError_t aria_k_pingpong(float *x, const float *v, const float *noise, float t
                            size_t n, hipStream_t s);
 /* fp32 -> fp16 (RTNE), n elements. */
 hipError_t aria_k_f32_to_f16(uint16_t *y, const float *x, size_t n, hipStream_t s);
-/* per batch b: dst[b] [cols, rows] = transpose of src[b] [rows, cols] */
-hipError_t aria_k_transpose(float *dst, const float *src, int rows, int cols, int batch, hipStream_t s);
-/* the same of src + add (add NULL: src alone), stored to dst and, unless it is NULL, dst2 */
+/* per batch b: dst[b] [cols, rows] = transpose of src[b] + add[b] [rows, cols] (add NULL: src alone),
+ * stored to dst and, unless it is NULL, dst2 */
 hipError_t aria_k_transpose2(float *dst, float *dst2, const float *src, const float *add, int rows, int cols, int batch,
                              hipStream_t s);
 /* dst + b * dst_stride [n] = src [n] for b < batch (n a multiple of 4, 16-byte aligned) */

@@ -27,7 +27,6 @@
 #define DEC_D 768
 #define DEC_S 34
 #define DEC_HD 64
-#define DEC_RH 16           /* rot / 2 */
 #define DEC_QKV 3840
 
 /* xt[t][c] = half(latent[c][t] * std): 64 x 4 tiles through LDS (coalesced on both sides) */

@@ -321,9 +321,6 @@ extern "C" hipError_t aria_k_transpose2(float *dst, float *dst2, const float *sr
     hipLaunchKernelGGL(k_transpose, grid, dim3(256), 0, s, dst, dst2, src, add, rows, cols);
     return hipGetLastError();
 }
-extern "C" hipError_t aria_k_transpose(float *dst, const float *src, int rows, int cols, int batch, hipStream_t s) {
-    return aria_k_transpose2(dst, nullptr, src, nullptr, rows, cols, batch, s);
-}
 
 /* one source row set to every sequence of a batch (the DiT's memory tokens in front of each): one
  * launch of ~2 us where a device copy per sequence took ~5 us each */

@@ -390,7 +390,9 @@ static int pick_wr(int M, int N, int K) {
  * HEADS 1.6-1.9x faster than those configurations in the geometric mean and are within 1-2 % of
  * the fastest of each shape on average (fp16 4 %). Down to two rows of tiles the small tiles of
  * k_qgemm_ks.hip win because they give every CU work; from about M = 860 (N = 8192) to 1420
- * (N = 1024) on, the large tiles' fewer bytes per product do. */
+ * (N = 1024) on, the large tiles' fewer bytes per product do. (fp16 outside HEADS has no fit for
+ * the 96 x 64 and the two-per-CU 64 x 64 K-split tiles: of 308 shapes, the decoder's among them, 20 would
+ * run 3-20 % faster on one of them than on their pick, none of the decoder's at M = 1870 or 11016.) */
 struct TileCost { int pick, bm, bn; float c0, c1, ck, co; };
 static const TileCost cost_q8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 1.4f}, {GEMM_KS + 1, 32, 64, 1.2f, 1.7f, 2.0f},
     {GEMM_KS + 2, 64, 64, 1.3f, 3.2f, 2.6f}, {GEMM_KS + 3, 96, 64, 2.0f, 3.9f, 3.2f}, {GEMM_KS + 4, 64, 64, 2.9f, 0.6f, 3.4f},
@@ -551,7 +553,8 @@ static hipError_t launch_q(const QArgs &a, int tiles, hipStream_t s) {
         hipLaunchKernelGGL((k_qgemm_simt<WT, AF16>), grid, dim3(256), 0, s, a);
         return hipGetLastError();
     }
-    if constexpr (!AF16) {   /* fp32 activations: the fallback when no fp16 staging buffer was available */
+    if constexpr (!AF16) {   /* fp32 activations: the K-split kernel where it takes them as they are, else (no
+                              * fp16 staging buffer, or none used: the step's io projections) 128 x 128 tiles */
         if (a.epi.mode == ARIA_EPI_HEADS) return hipErrorInvalidValue;
         if (tiles >= GEMM_KS) return qgemm_ks_f32_launch(a, WT, tiles - GEMM_KS, s);
         const bool plain = !a.gelu && (a.epi.mode == ARIA_EPI_STORE || a.epi.mode == ARIA_EPI_ADD);

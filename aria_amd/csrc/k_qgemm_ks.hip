@@ -1,24 +1,28 @@
 /*
  * k_qgemm_ks.hip - the GEMM for few output tiles (gfx950 MFMA): y[M,N] = x[M,K] W[N,K]^T (+ b)
  * for Q8 / Q4 / fp16 weights with fp16 activations and the W8A8 int8 form, with every fused
- * epilogue, K % 64 == 0.
+ * epilogue, K % 64 == 0 (int8: K % 128 == 0).
  * Replaces the same reference functions as k_qgemm.hip (aria_linear_q8 / aria_linear_q4,
  * src/aria_quant.c:98-145, 469-538; aria_linear_q8a8, src/aria_quant.c:253-345).
  *
  * A short sequence leaves the large-tile kernel (k_qgemm_big.hip) a handful of workgroups, each
  * walking the whole K range with a barrier per K-tile: the launch is one long latency chain on a
  * few CUs. Here a workgroup of KW waves owns one small tile of 32 FM x 32 FN outputs and the
- * waves split K between them: wave w takes the 64-byte K-tiles w, w + KW, ... on a pipeline of its
- * own (NST stages of LDS that no other wave touches), so the main loop has no barrier at all and
- * KW * (NST - 1) K-tiles are in flight per workgroup at any time. The partial sums then meet in
+ * waves split K between them: wave w takes the K-tiles w, w + KW, ... (RB bytes of each activation
+ * row) on a pipeline of its own (NST stages of LDS that no other wave touches), so the main loop has
+ * no barrier at all. While a wave waits for a K-tile, NST - 1 later ones are in flight; it reads the
+ * tile into registers, sends for tile + NST into the same stage, and multiplies. NST is what fits the
+ * LDS, up to four (KCfg): 2 or 3 in most configurations, 1 with fp16 or int8 weights in configuration
+ * 1, whose next tile then travels only while the last one is multiplied. The partial sums then meet in
  * LDS once, each element added in wave order (a fixed order: the same bits every launch; int32
  * exactly), and every wave finalises its share of the rows with the fused epilogue.
  *
  * Operands travel HBM -> LDS by LDS DMA (global_load_lds_dwordx4) and come back as MFMA
- * fragments; Q8 and Q4 are unpacked in registers. A K-tile is 64 bytes of every activation row:
- * 32 fp16 or 64 int8. Its 16-byte chunk c holds k [8c, 8c + 8) (int8: [16c, 16c + 16)); MFMA step s
- * of lane half h takes chunk 2 h + s on both sides, so a lane's Q8 weights of a K-tile are 16
- * contiguous bytes and its Q4 weights 8 (all in one quantization block).
+ * fragments; Q8 and Q4 are unpacked in registers. A K-tile is RB = 128 (configuration 4: 64) bytes
+ * of every activation row: KK = RB / 2 fp16, RB int8 or RB / 4 fp32 values, NK MFMA steps. Its 16-byte
+ * chunk c holds k [8c, 8c + 8) (int8: [16c, 16c + 16); fp32: [4c, 4c + 4)); step s of lane half h takes
+ * chunk NK h + s on both sides (fp32 activations: the two chunks of its eight k), so a lane's Q8
+ * weights of a K-tile are 8 NK contiguous bytes and its Q4 weights 4 NK (all in one quantization block).
  *
  * Order of the tiles: an XCD's contiguous run goes down the rows of one weight panel first
  * (N-major), so a weight panel comes from HBM into one XCD's L2; the few activation rows are what

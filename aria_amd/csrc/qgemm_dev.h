@@ -472,7 +472,7 @@ hipError_t qgemm_big_i8_launch(const QArgs &a, int cfg, hipStream_t s);
 int qgemm_big_i8_ncfg();
 
 /* the K-split kernel's launcher (k_qgemm_ks.hip): configuration cfg of qgemm_ks_ncfg(); wt is
- * ARIA_WQ8, ARIA_WQ4, ARIA_WF16 (fp16 activations) or ARIA_WI8 (int8 ones), K % 64 == 0 */
+ * ARIA_WQ8, ARIA_WQ4, ARIA_WF16 (fp16 activations, K % 64 == 0) or ARIA_WI8 (int8 ones, K % 128 == 0) */
 hipError_t qgemm_ks_launch(const QArgs &a, int wt, int cfg, hipStream_t s);
 int qgemm_ks_ncfg();
 /* the same with fp32 activations, rounded to fp16 as fragments are read (configurations 0 .. 2,

@@ -144,7 +144,7 @@ int aria_hip_qlinear_dev(void *dy, int y_f16, const void *dx, int x_f16, int wty
  * (both operands staged through LDS); 9..12 = 32x256, 64x256, 96x256, 128x256 with the
  * weights loaded straight into registers (Q8/Q4 with K % 64 == 0, else the 128x128 LDS
  * kernel); 0 = chosen from the shape (tuning knob; fp32 activations without an fp16
- * staging buffer always run 128x128). */
+ * staging buffer run 128x128, or with tiles 0 and few outputs the K-split kernel). */
 int aria_hip_qlinear_ex_dev(void *dy, int y_f16, const void *dx, int x_f16, int wtype, const void *dq,
                             const float *dscale, const float *db, int M, int K, int N, int tiles,
                             void *stream);
