@@ -392,7 +392,7 @@ static int pick_wr(int M, int N, int K) {
  * k_qgemm_ks.hip win because they give every CU work; from about M = 860 (N = 8192) to 1420
  * (N = 1024) on, the large tiles' fewer bytes per product do. (fp16 outside HEADS has no fit for
  * the 96 x 64 and the two-per-CU 64 x 64 K-split tiles: of 308 shapes, the decoder's among them, 20 would
- * run 3-20 % faster on one of them than on their pick, none of the decoder's at M = 1870 or 11016.) */
+ * run 3-20 % faster on one of them than on their pick, none of the decoder's from M = 1836 on.) */
 struct TileCost { int pick, bm, bn; float c0, c1, ck, co; };
 static const TileCost cost_q8[] = {{GEMM_KS, 32, 32, 1.0f, 1.6f, 1.4f}, {GEMM_KS + 1, 32, 64, 1.2f, 1.7f, 2.0f},
     {GEMM_KS + 2, 64, 64, 1.3f, 3.2f, 2.6f}, {GEMM_KS + 3, 96, 64, 2.0f, 3.9f, 3.2f}, {GEMM_KS + 4, 64, 64, 2.9f, 0.6f, 3.4f},
